@@ -155,6 +155,13 @@ constexpr bool kDmaDown = true;
 
 }  // namespace
 
+// 64-row tasks of shapes outside the tuned kernels: the LDS-tiled kernels
+// (E = 32, H = I = 2880, T = 512: 312 us per layer against 768 with the
+// run-time-K kernels; E = 128, H = 2048, I = 96, T = 1024: 76 against 113)
+// except for matrices so small that the stage ring's start costs more than the
+// products (H = 96, I = 32: 19.5 against 17.2 us).
+static bool generic_tiled(int H, int I) { return tile_gemm_ok(H, I) && (long long)H * I >= 65536; }
+
 hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_block, bool w4,
                           int path, int num_cus, hipStream_t s) {
   // W4 with several rows per expert, and every 64-row task: decode each weight
@@ -165,7 +172,7 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   const bool wave_ok = w4 && wave_w4_shape_ok(a.H, a.I, token_block);
   if (wave_ok && path != kGeneric && (token_block == 64 || ((long long)a.R >= 4LL * a.E && !a.w4_fold)))
     return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (path == kTile) return w4 ? hipErrorInvalidValue : launch_tile_gate_up(a, task_capacity, num_cus, s);
+  if (path == kTile) return w4 ? hipErrorInvalidValue : launch_tile_gate_up(a, num_cus, s);
   if (path == kStream) {
     if (!w4 && kDmaStreaming && dma_shape_ok(a.H, a.I, token_block))
       return launch_dma_gate_up(a, token_block, num_cus, s);
@@ -175,6 +182,8 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   // fit, else the run-time-K MFMA kernel, else (bf16, H or I not a multiple of
   // 32) the scalar one.
   if (wave_ok) return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
+  if (path == kGeneric && token_block == 64 && !w4 && generic_tiled(a.H, a.I))
+    return launch_tile_gate_up(a, num_cus, s);
   if (path == kGeneric && flex_shape_ok(a.H, a.I, w4))
     return launch_flex_gate_up(a, task_capacity, token_block, w4, s);
   if (w4) return hipErrorInvalidValue;
@@ -185,11 +194,13 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
 
 hipError_t launch_down(const ExpertArgs &a, int task_capacity, int token_block, int path,
                        int num_cus, hipStream_t s) {
-  if (path == kTile) return launch_tile_down(a, task_capacity, num_cus, s);
+  if (path == kTile) return launch_tile_down(a, num_cus, s);
   if (path == kStream) {
     if (kDmaStreaming && kDmaDown && dma_shape_ok(a.H, a.I, token_block)) return launch_dma_down(a, token_block, num_cus, s);
     return launch_stream_down(a, task_capacity, token_block, num_cus, s);
   }
+  if (path == kGeneric && token_block == 64 && generic_tiled(a.H, a.I))
+    return launch_tile_down(a, num_cus, s);
   if (path == kGeneric && flex_shape_ok(a.H, a.I, false))
     return launch_flex_down(a, task_capacity, token_block, s);
   const dim3 grid(task_capacity, (token_block * a.H + 255) / 256);

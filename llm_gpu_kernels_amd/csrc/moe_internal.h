@@ -91,14 +91,17 @@ hipError_t launch_dma_gate_up_planned(const ExpertArgs &a, const RouteArgs &ra, 
 bool wave_w4_shape_ok(int H, int I, int token_block);
 hipError_t launch_wave_w4_gate_up(const ExpertArgs &a, int task_capacity, int token_block,
                                   hipStream_t s);
-hipError_t launch_tile_gate_up(const ExpertArgs &a, int task_capacity, int num_cus,
-                               hipStream_t s);
-hipError_t launch_tile_down(const ExpertArgs &a, int task_capacity, int num_cus, hipStream_t s);
+// LDS-tiled bf16 GEMMs for many rows per expert (64-row tasks), moe_tile.hip.
+hipError_t launch_tile_gate_up(const ExpertArgs &a, int num_cus, hipStream_t s);
+hipError_t launch_tile_down(const ExpertArgs &a, int num_cus, hipStream_t s);
+bool tile_gemm_ok(int H, int I);
+// Shapes that report the tiled family (moe_layout.fast_path 2).
 bool tile_shape_ok(int H, int I, bool w4);
 
 // Expert-stage kernel families (moe_layout.fast_path).
-// kGeneric: the run-time-K MFMA kernels (or scalar kernels where H or I is not
-// a multiple of 32); kScalar: the scalar kernels (unaligned bf16 buffers).
+// kGeneric: the run-time-K MFMA kernels, with 64-row tasks the tiled bf16
+// kernels where tile_gemm_ok (or scalar kernels where H or I is not a multiple
+// of 32); kScalar: the scalar kernels (unaligned bf16 buffers).
 enum Path { kGeneric = 0, kStream = 1, kTile = 2, kScalar = 3 };
 // MFMA kernels for any H, I that are multiples of 32 (W4: H of 128) -- the
 // shapes the tuned kernels above do not take (kGeneric path).

@@ -1,23 +1,24 @@
 // LDS-tiled grouped GEMMs of the MoE forward on gfx950 for large row counts.
 //
-// When experts receive many rows (T = 1024, Zipf-skewed routing: a few
-// experts take ~1000 rows), streaming each weight byte once per 16/32-row task
-// would re-read the hot experts' weights dozens of times.  Here a task holds
-// up to BM = 64 grouped rows and a work unit is (task, n-tile of BN weight
-// rows); units are numbered expert-major and n-tile-major within an expert,
-// and that sequence is cut into one contiguous chunk per XCD, so the tasks of
-// an expert that share a weight tile, and the n-tiles of a task that share its
-// token rows, are read through one XCD's L2 (HBM reads at T = 1024 Zipf:
-// gate/up 765 -> 661 MB, down 382 -> 312 MB, against 4-task blocks dealt
-// round-robin).
+// When experts receive many rows (prefill chunks, skewed routing), streaming
+// each weight byte once per 16/32-row task would re-read the hot experts'
+// weights dozens of times.  Here a work unit is (expert, block of up to 160 of
+// its grouped rows, tile of 256 weight rows).  An expert's rows are cut into
+// the fewest such blocks, of equal height (a multiple of 32), taken from
+// counts[] and offsets[]: the planner's 64-row task list is not used, only its
+// length (zero when the plan stalled).  Units are numbered expert-major and
+// weight-tile-major within an expert, and that sequence is cut into one
+// contiguous chunk per XCD, so the row blocks that share a weight tile, and
+// the weight tiles that share a block's token rows, meet in one XCD's L2.
 //
-// Per unit: a K loop over BK-wide stages.  Each stage's weight tile [BN][BK]
-// and token tile [BM][BK] go global -> LDS (the warp-specialised kernel
-// below), 16-byte chunks XOR-swizzled by row so that the MFMA operand reads
-// are bank-conflict free, then 8 waves (4 along N x 2 along M) run 16x16x32
-// bf16 MFMAs.  (W4G128 gate/up with many rows per expert runs in
-// the wave kernel of moe_wave.hip, which decodes each weight once into MFMA
-// registers; the down weights are bf16 in both formats.)
+// Per unit: a K loop over 64-wide stages.  Each stage's weight tile [256][64]
+// and token tile [32 nb][64] go global -> LDS with buffer loads that write LDS
+// directly (16-byte chunks XOR-swizzled by row on the global side, so that the
+// MFMA operand reads are bank-conflict free).  The descriptors are bounded at
+// the expert's matrix: weight rows past I or H, and the chunks of the last
+// stage past K, read as zero, so any H and I that are multiples of 32 run
+// here.  (W4G128 gate/up with many rows per expert runs in the wave kernel of
+// moe_wave.hip; the down weights are bf16 in both formats.)
 //
 // Epilogues match the streaming kernels: gate/up round to bf16, SwiGLU in
 // fp32, bf16 act rows; down rounds to bf16 and scatters rows to route order.
@@ -25,12 +26,11 @@
 #include "moe_internal.h"
 
 #define MOE_CONST __attribute__((address_space(4)))
+#define MOE_LDS __attribute__((address_space(3)))
 
 namespace moe {
 
 namespace {
-
-constexpr int BM = 64;
 
 template <typename T>
 __device__ __forceinline__ const MOE_CONST T *as_const(const T *p) {
@@ -43,38 +43,40 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Byte offset of 16-byte chunk c of row `row` in a [rows][BK] bf16 tile.
-template <int BK>
-__device__ __forceinline__ int swz(int row, int c) {
-  if constexpr (BK == 64) return row * 128 + ((c ^ ((row >> 1) & 7)) << 4);
-  else return row * 256 + ((c ^ (row & 15)) << 4);
+__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
 
-
-template <int KIND>
-struct TileCfg {
-  static constexpr int BN = 256;  // weight rows per tile
-  static constexpr int BK = 64;
-  static constexpr int WNT = BN / 4 / 16;                   // 16-row tiles per wave
-  static constexpr int A_BYTES = BN * BK * 2;
-  static constexpr int B_BYTES = BM * BK * 2;
-  static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-  static constexpr int OUT_COLS = KIND == 0 ? BN / 2 : BN;  // output columns per n-tile
-};
-
-// ---- warp-specialised kernel ---------------------------------------------------
-// The K stages move by global -> LDS direct loads (16 bytes per lane, gfx950)
-// into a ring of kWsStages LDS stages, kWsStages - 1 stages ahead of the
-// matrix cores.  Four loader waves
-// issue every load and carry every vector-memory wait; the eight MFMA waves
-// only read LDS.  One workgroup barrier per stage publishes that stage (the
-// loaders waited for it) and frees the oldest buffer (every MFMA wave has
-// finished reading it).  One 768-thread workgroup per CU owns all 160 KB of
-// LDS.
-constexpr int kWsConsumers = 8;
-constexpr int kWsLoaders = 4;
-constexpr int kWsThreads = (kWsConsumers + kWsLoaders) * 64;
-constexpr int kWsStages = 4;
+// ---- shape of the kernel -------------------------------------------------------
+// One 512-thread workgroup per CU: four MFMA waves, one per SIMD, and four
+// loader waves, so each may use 256 VGPRs.  MFMA wave w owns 64 weight rows
+// (gate/up: 32 gate and the 32 up rows of the same features) against all of
+// the block's token rows: 2 x nb tiles of 32 x 32, at most 160 accumulator
+// registers.  Per 16-K step it reads 2 + nb operand fragments for 2 nb MFMAs
+// and reads each step's fragments before the MFMAs of the step before, across
+// stage boundaries too.  The loader waves issue every global load and carry
+// every vector-memory wait; one workgroup barrier per stage publishes that
+// stage (the loaders waited for it) and frees the oldest slot of the ring.
+//
+// Measured at E = 128, H = 2048, I = 768, K = 8 against 64-row tasks with 64 x
+// 32 wave tiles and every fragment of a stage read before its MFMAs: T = 4096
+// gate/up 350 -> 237 us, down 215 -> 146 us; T = 1024 Zipf 153 -> 137 and 92 ->
+// 80 us.  At T = 4096 the loads alone take 188 us (2.5 GB through L2, 966 MB of
+// HBM reads, 5.1 TB/s), the MFMAs and LDS reads alone 111 us, the epilogues 27.
+constexpr int kBN = 256;                // weight rows per tile
+constexpr int kBK = 64;                 // K per stage: one 128-byte piece per row
+constexpr int kMaxNB = 5;               // 32-row token blocks per unit
+constexpr int kABytes = kBN * kBK * 2;
+constexpr int kRingBytes = (int)kMaxLds;
+// Ring slots for units of up to NBM token blocks: three of 52 KiB, or four of
+// 40 KiB (three stages in flight) where no unit is higher than 64 rows.
+constexpr int slot_bytes(int NBM) { return kABytes + NBM * 32 * kBK * 2; }
+constexpr int ring_slots(int NBM) { return kRingBytes / slot_bytes(NBM); }
+constexpr int kMfmaWaves = 4;
+constexpr int kLoaders = 4;
+constexpr int kThreads = (kMfmaWaves + kLoaders) * kWave;
+constexpr int kAPer = kBN / kLoaders / 8;  // weight loads per loader wave and stage
+static_assert(ring_slots(2) == 4 && ring_slots(kMaxNB) == 3, "the loaders' wait counts cover three and four slots");
 
 // s_waitcnt with only the vector-memory counter bounded (gfx9 encoding).
 template <int N>
@@ -82,263 +84,451 @@ __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
+// At most n vector-memory operations outstanding (n wave-uniform: the loads of
+// one or two stages, or 0).
+__device__ __forceinline__ void wait_vmcnt_upto(int n) {
+  switch (n) {
+#define MOE_W(N) case N: wait_vmcnt<N>(); break;
+    MOE_W(9) MOE_W(10) MOE_W(11) MOE_W(12) MOE_W(13)   // one stage
+    MOE_W(18) MOE_W(19) MOE_W(20)                       // two stages of one or two token blocks
+#undef MOE_W
+    default: wait_vmcnt<0>(); break;
+  }
+}
 
-template <int KIND>
-__global__ __launch_bounds__(kWsThreads) void tile_ws_kernel(ExpertArgs a) {
-  using C = TileCfg<KIND>;
-  constexpr int BN = C::BN, BK = C::BK, WNT = C::WNT;
-  constexpr int KS = BK / 32;
-  static_assert(BK == 64, "one 128-byte row piece per stage");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+// 16 bytes per lane from a buffer straight into LDS (lane l's bytes at
+// dst + 16 l); lanes whose voff is past the descriptor's size write zeros
+// (soff is not part of that check).  Device pass only, as in the attention.
+__device__ __forceinline__ void buffer_load_lds16(__amdgpu_buffer_rsrc_t rs, uint8_t *dst, uint32_t voff,
+                                                  uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (MOE_LDS void *)dst, 16, voff, soff, 0, 0);
+#endif
+}
 
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int H = a.H, I = a.I;
-  const int Kdim = KIND == 0 ? H : I;
-  const int KT = Kdim / BK;
-  const int ntiles = (KIND == 0 ? I : H) / C::OUT_COLS;
-  const int num_tasks = *as_const(a.num_tasks);
-  const int total = num_tasks * ntiles;
-  const MOE_CONST int32_t *tasks = as_const((const int32_t *)a.tasks);
-  const int G = gridDim.x;
-  // XCD-affine order: the unit sequence, expert-major and n-tile-major
-  // within an expert (every task of the expert on one n-tile, then the next
-  // n-tile), is cut into eight contiguous chunks, one per XCD (consecutive
-  // workgroup IDs go round-robin over the XCDs), and the workgroups of an XCD
-  // walk their chunk together.  So an expert's weight tile and its tasks'
-  // token rows are read from one XCD's L2, except at the seven chunk edges.
-  const bool xcd_mode = G % 8 == 0 && G >= 8;
-  const int P = xcd_mode ? G / 8 : G;            // workgroups per XCD
-  const int xcd = xcd_mode ? (int)blockIdx.x % 8 : 0;
-  const int p = xcd_mode ? (int)blockIdx.x / 8 : (int)blockIdx.x;
-  const int CH = xcd_mode ? (total + 7) / 8 : total;  // units per chunk
-  const int c_end = min(CH, total - xcd * CH);
-  const int nu = p < c_end ? (c_end - p + P - 1) / P : 0;
-  const MOE_CONST int32_t *cnts = as_const(a.counts);
-  const MOE_CONST int32_t *offs = as_const(a.offsets);
-  const int nstages = nu * KT;
+__device__ __forceinline__ int sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-  struct Unit {
-    int e, row0, rows, nt;
-  };
-  auto unit_of = [&](int i) {
-    const int L = xcd * CH + p + i * P;
-    const int T = L / ntiles;  // the task whose expert owns unit L
-    const int e = tasks[4 * T];
-    const int t0 = T - (tasks[4 * T + 1] - offs[e]) / BM;  // the expert's first task
-    const int m = (cnts[e] + BM - 1) / BM;                 // and its task count
-    const int local = L - ntiles * t0;
-    Unit un;
-    un.nt = local / m;
-    const int t = t0 + (local - un.nt * m);
-    un.e = e;
-    un.row0 = tasks[4 * t + 1];
-    un.rows = tasks[4 * t + 2];
-    return un;
-  };
+// The unit sequence, held by every wave: lane l has the row counts and first
+// grouped rows of experts 4 l .. 4 l + 3 and the number of units before them.
+struct UnitMap {
+  int cnt[4], off[4];
+  int before;
+  int total;
+  int ntiles;
+  uint32_t max_rows;  // rows per unit at most (a multiple of 32)
 
-  if (wave >= kWsConsumers) {
-    // ---- loaders: wave lw moves tile rows [lw*64, +64) of the weights and
-    // [lw*16, +16) of the tokens, 8 rows (1 KiB of LDS) per instruction.
-    const int lw = wave - kWsConsumers;
-    constexpr int A_PER = BN / kWsLoaders / 8;
-    constexpr int B_PER = BM / kWsLoaders / 8;
-    constexpr int PER = A_PER + B_PER;  // instructions per stage per loader wave
-    static_assert(kWsStages == 4 && 2 * PER < 64, "wait counts below assume 4 stages");
-    const uint16_t *asrc[A_PER];
-    const uint16_t *bsrc[B_PER];
-    int cur = -1;
-    auto setup = [&](int i) {
-      const Unit un = unit_of(i);
+  __device__ __forceinline__ int blocks(int n) const { return (int)(((uint32_t)n + max_rows - 1) / max_rows); }
+
+  __device__ __forceinline__ void init(const int32_t *counts, const int32_t *offsets, int E, int nt, int rows,
+                                       int lane) {
+    ntiles = nt;
+    max_rows = (uint32_t)rows;
+    int mine = 0;
 #pragma unroll
-      for (int j = 0; j < A_PER; ++j) {
-        const int row = lw * (BN / kWsLoaders) + j * 8 + lane / 8;  // tile row
-        const int c = (lane % 8) ^ ((row >> 1) & 7);  // logical chunk of LDS chunk lane%8
-        size_t wrow;
-        if (KIND == 0)
-          wrow = (size_t)un.e * 2 * I +
-                 (row < BN / 2 ? un.nt * (BN / 2) + row : I + un.nt * (BN / 2) + row - BN / 2);
-        else
-          wrow = (size_t)un.e * H + un.nt * BN + row;
-        asrc[j] = (KIND == 0 ? a.gate_up : a.down) + wrow * Kdim + c * 8;
-      }
-      // Token of each B row through scalar loads (the loaders' vector-memory
-      // counter then holds only their LDS loads, so nothing here waits on
-      // them); rows past the task's end take the task's first token.
-      constexpr int BR = BM / kWsLoaders;  // B rows of this loader wave
-      int tokv[BR];
-      if (KIND == 0) {
-        const MOE_CONST int32_t *rt = as_const(a.row_token) + un.row0;
-        const int t0 = rt[0];
-#pragma unroll
-        for (int k = 0; k < BR; ++k) tokv[k] = lw * BR + k < un.rows ? rt[lw * BR + k] : t0;
-      }
-#pragma unroll
-      for (int j = 0; j < B_PER; ++j) {
-        const int row = lw * BR + j * 8 + lane / 8;
-        const int c = (lane % 8) ^ ((row >> 1) & 7);
-        size_t off;
-        if (KIND == 0) {
-          int tok = tokv[j * 8];
-#pragma unroll
-          for (int k = 1; k < 8; ++k) tok = lane / 8 == k ? tokv[j * 8 + k] : tok;
-          off = (size_t)tok * H;
-        } else {
-          off = (size_t)(un.row0 + (row < un.rows ? row : 0)) * I;
-        }
-        bsrc[j] = (KIND == 0 ? a.x : a.act) + off + c * 8;
-      }
-    };
-    auto issue = [&](int st) {
-      const int i = st / KT, kt = st - (st / KT) * KT;
-      if (i != cur) {
-        setup(i);
-        cur = i;
-      }
-      uint8_t *buf = smem + (st % kWsStages) * C::STAGE_BYTES;
-#pragma unroll
-      for (int j = 0; j < A_PER; ++j)
-        __builtin_amdgcn_global_load_lds(
-            (const void *)(asrc[j] + kt * BK),
-            (__attribute__((address_space(3))) void *)(buf + (lw * (BN / kWsLoaders) + j * 8) * 128),
-            16, 0, 0);
-#pragma unroll
-      for (int j = 0; j < B_PER; ++j)
-        __builtin_amdgcn_global_load_lds(
-            (const void *)(bsrc[j] + kt * BK),
-            (__attribute__((address_space(3))) void *)(buf + C::A_BYTES +
-                                                       (lw * (BM / kWsLoaders) + j * 8) * 128),
-            16, 0, 0);
-    };
-    for (int st = 0; st < kWsStages - 1 && st < nstages; ++st) issue(st);
-    for (int st = 0; st < nstages; ++st) {
-      // Stage st has landed once at most the loads issued after it remain.
-      const int later = min(kWsStages - 2, nstages - 1 - st);
-      if (later >= 2) wait_vmcnt<2 * PER>();
-      else if (later == 1) wait_vmcnt<PER>();
-      else wait_vmcnt<0>();
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      // Buffer (st - 1) % stages was last read before this barrier.
-      if (st + kWsStages - 1 < nstages) issue(st + kWsStages - 1);
+    for (int j = 0; j < 4; ++j) {
+      const int e = min(4 * lane + j, E - 1);
+      cnt[j] = counts[e];
+      off[j] = offsets[e];
     }
-    return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      cnt[j] = 4 * lane + j < E ? cnt[j] : 0;
+      mine += blocks(cnt[j]) * nt;
+    }
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int up = __shfl_up(incl, o, kWave);
+      if (lane >= o) incl += up;
+    }
+    before = incl - mine;
+    total = __builtin_amdgcn_readlane(incl, kWave - 1);
   }
 
-  // ---- MFMA waves: (wn, wm) = 64 weight rows x 32 tokens ------------------
-  const int wn = wave & 3, wm = wave >> 2;
-  auto a_row = [&](int i) {
-    if (KIND == 0) {
-      constexpr int HALF_T = WNT / 2;
-      return (i < HALF_T ? 0 : BN / 2) + wn * HALF_T * 16 + (i % HALF_T) * 16;
-    }
-    return wn * WNT * 16 + i * 16;
+  struct Unit {
+    int e, row0, rows, nt;  // expert, first grouped row, rows, weight tile
   };
-  int st = 0;
-  for (int i = 0; i < nu; ++i) {
-    const Unit un = unit_of(i);
-    f32x4 acc[WNT][2];
+  __device__ __forceinline__ Unit at(int u) const {
+    // The last lane whose experts start at or before u.
+    const int src = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before <= u)) - 1;
+    int local = u - __builtin_amdgcn_readlane(before, src);
+    Unit un;
+    un.e = 4 * src;
+    int n = __builtin_amdgcn_readlane(cnt[0], src), o = __builtin_amdgcn_readlane(off[0], src);
 #pragma unroll
-    for (int q = 0; q < WNT; ++q) acc[q][0] = acc[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kt = 0; kt < KT; ++kt, ++st) {
-      lds_barrier();  // stage st published; every read of stage st - 1 is done
-      const uint8_t *abuf = smem + (st % kWsStages) * C::STAGE_BYTES;
-      const uint8_t *bbuf = abuf + C::A_BYTES;
-      const int r = lane & 15, g = lane >> 4;
-      // Every fragment of the stage is requested before the first MFMA, so
-      // the stage costs one LDS round trip.
-      u32x4 bf[KS][2], af[KS][WNT];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int c = 4 * ks + g;
-        bf[ks][0] = *(const u32x4 *)(bbuf + swz<BK>(wm * 32 + r, c));
-        bf[ks][1] = *(const u32x4 *)(bbuf + swz<BK>(wm * 32 + 16 + r, c));
-#pragma unroll
-        for (int q = 0; q < WNT; ++q) af[ks][q] = *(const u32x4 *)(abuf + swz<BK>(a_row(q) + r, c));
-      }
-      __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int q = 0; q < WNT; ++q) {
-          acc[q][0] = mfma16(af[ks][q], bf[ks][0], acc[q][0]);
-          acc[q][1] = mfma16(af[ks][q], bf[ks][1], acc[q][1]);
-        }
+    for (int j = 1; j < 4; ++j) {
+      const int sz = blocks(n) * ntiles;
+      const bool past = un.e == 4 * src + j - 1 && local >= sz;
+      const int nn = __builtin_amdgcn_readlane(cnt[j], src), on = __builtin_amdgcn_readlane(off[j], src);
+      local -= past ? sz : 0;
+      un.e += past ? 1 : 0;
+      n = past ? nn : n;
+      o = past ? on : o;
     }
-    // Epilogue (registers only, no LDS): lane holds rows 4*(l/16)+k of its
-    // 16-row weight tile for token l%16.
-    const int g = lane >> 4;
+    const int m = blocks(n);
+    un.nt = local / m;
+    const int b = local - un.nt * m;
+    const int per = ((n + m - 1) / m + 31) & ~31;  // equal heights, whole 32-row blocks
+    un.row0 = o + b * per;
+    un.rows = min(per, n - b * per);
+    return un;
+  }
+};
+
+// SiLU(g) * u in fp32: g / (1 + e^-g) * u with the hardware's base-2 exponential
+// and reciprocal (about 1 ulp each; the product is rounded to bf16).
+__device__ __forceinline__ float swiglu(float g, float u) {
+  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * g);
+  return g * __builtin_amdgcn_rcpf(1.0f + e) * u;
+}
+
+// Streaming stores: act and routed rows are read by the next launch only, and
+// lines left dirty in L2 (up to 32 MiB over the XCDs) are written back at the
+// end of the kernel, when nothing else runs (down at T = 1024: 87 -> 79 us).
+__device__ __forceinline__ void store_row(uint16_t *p, u32x4 v) { __builtin_nontemporal_store(v, (u32x4 *)p); }
+
+// Weight row within a 32-row fragment that LDS row m of it holds: the MFMA
+// leaves output rows 8 q + 4 h + i (q, i = 0..3) in lane half h, so with this
+// order a lane's sixteen outputs are sixteen consecutive columns.
+__device__ __forceinline__ int frag_row(int m) { return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3); }
+
+template <int KIND, int NBM>
+__device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &map, int first, int stride, int nu,
+                                          int lw, int lane, uint8_t *smem) {
+  constexpr int kSlots = ring_slots(NBM), kSlotBytes = slot_bytes(NBM);
+  const int H = a.H, I = a.I;
+  const int Kdim = KIND == 0 ? H : I;
+  const int KT = (Kdim + kBK - 1) / kBK;
+  const int nstages = nu * KT;
+  const uint32_t pitch = (uint32_t)Kdim * 2u;
+  const uint32_t tail = (uint32_t)(Kdim % kBK) / 8u;  // 16-byte chunks in a partial last stage
+  const int lr = lane >> 3;
+
+  // Loader wave lw moves LDS rows [64 lw, +64) of the weight tile and rows
+  // 32 b + 8 lw .. + 8 of each token block, eight rows (1 KiB) per load.  LDS
+  // chunk lane % 8 of row r holds logical chunk (lane % 8) ^ ((r >> 1) & 7).
+  const uint8_t *xbase = KIND == 0 ? (const uint8_t *)a.x : (const uint8_t *)a.act;
+  const uint32_t xbytes = KIND == 0 ? (uint32_t)a.T * pitch : (uint32_t)a.R * pitch;
+  const auto brs = __builtin_amdgcn_make_buffer_rsrc((void *)xbase, (short)0, (int)xbytes, 0x00020000);
+  __amdgpu_buffer_rsrc_t ars;
+  uint32_t aoff[kAPer], boff[NBM];
+  // Rows r = 8 j + lr with j even or odd: (r >> 1) & 7 = 4 (j & 1) + lr / 2.
+  const uint32_t c0 = (uint32_t)((lane & 7) ^ (lr >> 1));  // j even; odd: ^ 4
+  int cur = -1, nb = 0;
+  auto setup = [&](int i) {
+    const UnitMap::Unit un = map.at(first + i * stride);
+    nb = (un.rows + 31) >> 5;
+    const size_t mat = (size_t)(KIND == 0 ? I : H) * pitch;  // one expert's gate, up or down matrix
+    const uint8_t *wb = KIND == 0 ? (const uint8_t *)a.gate_up + ((size_t)un.e * 2 + (lw >> 1)) * mat
+                                  : (const uint8_t *)a.down + (size_t)un.e * mat;
+    ars = __builtin_amdgcn_make_buffer_rsrc((void *)wb, (short)0, (int)(uint32_t)mat, 0x00020000);
+    // gate/up: LDS rows 0..127 are gate rows, 128..255 the up rows (the base above).
+    const int wrow0 = KIND == 0 ? un.nt * (kBN / 2) + (lw & 1) * 64 : un.nt * kBN + lw * 64;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int tok = wm * 32 + mt * 16 + (lane & 15);
+    for (int j = 0; j < kAPer; ++j) {
+      const int row = wrow0 + (j / 4) * 32 + frag_row((j & 3) * 8 + lr);
+      aoff[j] = (uint32_t)row * pitch + ((c0 ^ (4u * (j & 1))) << 4);
+    }
+    // Token of each row through scalar loads (the vector-memory counter holds
+    // only LDS loads, so nothing here waits on them); rows past the unit's
+    // end repeat its first row.
+    const MOE_CONST int32_t *rt = as_const(a.row_token) + un.row0;
+#pragma unroll
+    for (int b = 0; b < NBM; ++b) {
+      if (b >= nb) break;
+      const int r0 = b * 32 + lw * 8;
+      uint32_t off;
       if (KIND == 0) {
-        constexpr int HALF_T = WNT / 2;
+        const int t0 = rt[0];
+        int tok = t0;
 #pragma unroll
-        for (int q = 0; q < HALF_T; ++q) {
-          const f32x4 sg = acc[q][mt], su = acc[q + HALF_T][mt];
-          float v[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const float gt = bf16_round(sg[k]);
-            const float up = bf16_round(su[k]);
-            v[k] = gt / (1.0f + expf(-gt)) * up;
-          }
-          u32x2 packed;
-          packed[0] = pack_bf16x2(v[0], v[1]);
-          packed[1] = pack_bf16x2(v[2], v[3]);
-          const int col = un.nt * (BN / 2) + wn * HALF_T * 16 + q * 16 + 4 * g;
-          if (tok < un.rows) *(u32x2 *)(a.act + (size_t)(un.row0 + tok) * I + col) = packed;
+        for (int k = 0; k < 8; ++k) {
+          const int tk = r0 + k < un.rows ? rt[r0 + k] : t0;
+          tok = lr == k ? tk : tok;
         }
+        off = (uint32_t)tok * pitch;
       } else {
-        const int q0 = tok < un.rows ? a.row_route[un.row0 + tok] : 0;
-#pragma unroll
-        for (int q = 0; q < WNT; ++q) {
-          u32x2 packed;
-          packed[0] = pack_bf16x2(acc[q][mt][0], acc[q][mt][1]);
-          packed[1] = pack_bf16x2(acc[q][mt][2], acc[q][mt][3]);
-          const int col = un.nt * BN + wn * WNT * 16 + q * 16 + 4 * g;
-          if (tok < un.rows) *(u32x2 *)(a.routed + (size_t)q0 * H + col) = packed;
-        }
+        off = (uint32_t)(un.row0 + (r0 + lr < un.rows ? r0 + lr : 0)) * pitch;
       }
+      boff[b] = off + ((c0 ^ (4u * (lw & 1))) << 4);
+    }
+  };
+  int slot = 0, kt_next = 0, unit_next = 0;
+  // Issue stage (unit_next, kt_next); returns the loads issued.
+  auto issue = [&]() {
+    if (unit_next != cur) {
+      setup(unit_next);
+      cur = unit_next;
+    }
+    uint8_t *buf = smem + slot * kSlotBytes;
+    const uint32_t koff = (uint32_t)kt_next * (kBK * 2);
+    const bool part = tail != 0 && kt_next == KT - 1;
+    const uint32_t oe = part && c0 >= tail ? 0xffffffffu : 0u;         // chunks past K: out of range
+    const uint32_t oo = part && (c0 ^ 4u) >= tail ? 0xffffffffu : 0u;
+#pragma unroll
+    for (int j = 0; j < kAPer; ++j)
+      buffer_load_lds16(ars, buf + (lw * 64 + j * 8) * 128, aoff[j] | (j & 1 ? oo : oe), koff);
+    const uint32_t ob = lw & 1 ? oo : oe;
+#pragma unroll
+    for (int b = 0; b < NBM; ++b) {
+      if (b >= nb) break;
+      buffer_load_lds16(brs, buf + kABytes + (b * 32 + lw * 8) * 128, boff[b] | ob, koff);
+    }
+    slot = slot == kSlots - 1 ? 0 : slot + 1;
+    if (++kt_next == KT) {
+      kt_next = 0;
+      ++unit_next;
+    }
+    return kAPer + nb;
+  };
+  // Loads of the stages in flight behind stage st: st + 1 (and, with four
+  // slots, st + 2).
+  int n1 = 0, n2 = 0;
+  if (nstages > 0) issue();
+  if (nstages > 1) n1 = issue();
+  if (kSlots == 4 && nstages > 2) n2 = issue();
+  for (int st = 0; st < nstages; ++st) {
+    wait_vmcnt_upto(n1 + n2);  // stage st has landed
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    // The slot of stage st - 1 was last read before this barrier.
+    const int n = st + kSlots - 1 < nstages ? issue() : 0;
+    n1 = kSlots == 4 ? n2 : n;
+    n2 = kSlots == 4 ? n : 0;
+  }
+}
+
+// One unit on MFMA wave w with NB token blocks; `slot` is the ring slot of the
+// unit's first stage, returned advanced.
+template <int KIND, int NB, int NBM>
+__device__ __forceinline__ int mfma_unit(const ExpertArgs &a, const UnitMap::Unit &un, int KT, int slot, int w,
+                                         int lane, const uint8_t *smem) {
+  constexpr int kSlots = ring_slots(NBM), kSlotBytes = slot_bytes(NBM);
+  const int r = lane & 31, h = lane >> 5;
+  f32x16 acc[2][NB];
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[q][b][i] = 0.f;
+  // Down: route of each of this lane's rows, requested before the K loop (a
+  // load between the epilogue's stores would wait for them).
+  int route[NB];
+  if (KIND == 1) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) route[b] = 32 * b + r < un.rows ? a.row_route[un.row0 + 32 * b + r] : -1;
+  }
+  // Byte offset of this lane's chunk of K-step ks within a 32-row fragment.
+  uint32_t lo[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) lo[ks] = (uint32_t)(r * 128 + (((2 * ks + h) ^ ((r >> 1) & 7)) << 4));
+  const uint32_t a0 = KIND == 0 ? w * 4096 : w * 8192, a1 = KIND == 0 ? 16384 + w * 4096 : w * 8192 + 4096;
+
+  // One K-step: the MFMAs of the fragments read a step ago, with the next
+  // step's fragment reads issued between them.
+  u32x4 af[2][2], bf[2][NB];
+  auto read_one = [&](int set, const uint8_t *buf, int ks, int i) __attribute__((always_inline)) {
+    if (i == 0) af[set][0] = *(const u32x4 *)(buf + a0 + lo[ks]);
+    else if (i == 1) bf[set][0] = *(const u32x4 *)(buf + kABytes + lo[ks]);
+    else if (i == 2) af[set][1] = *(const u32x4 *)(buf + a1 + lo[ks]);
+    else if (i < NB + 2) bf[set][i - 2] = *(const u32x4 *)(buf + kABytes + (i - 2) * 4096 + lo[ks]);
+  };
+  auto read_all = [&](int set, const uint8_t *buf, int ks) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NB + 2; ++i) read_one(set, buf, ks, i);
+  };
+  auto step = [&](int set, const uint8_t *buf, int ks) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2 * NB; ++i) {
+      acc[i & 1][i >> 1] = mfma32(af[set][i & 1], bf[set][i >> 1], acc[i & 1][i >> 1]);
+      if (i < NB + 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        read_one(set ^ 1, buf, ks, i);
+        if (i == 2 * NB - 1)
+          for (int j = 2 * NB; j < NB + 2; ++j) read_one(set ^ 1, buf, ks, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  const uint8_t *buf = smem;
+  for (int kt = 0; kt < KT; ++kt) {
+    lds_barrier();  // the stage is published; every read of the stage before it is done
+    buf = smem + slot * kSlotBytes;
+    slot = slot == kSlots - 1 ? 0 : slot + 1;
+    if (kt == 0) read_all(0, buf, 0);
+    else step(1, buf, 0);
+    step(0, buf, 1);
+    step(1, buf, 2);
+    step(0, buf, 3);
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * NB; ++i) acc[i & 1][i >> 1] = mfma32(af[1][i & 1], bf[1][i >> 1], acc[i & 1][i >> 1]);
+
+  // Epilogue.  Lane (r, h) holds token row 32 b + r, columns 16 h .. + 16 of
+  // each fragment.  The rows go out through this wave's own weight rows of the
+  // last stage (8 KiB that only this wave reads, and that the loaders refill
+  // only after the next barrier), so that every store instruction writes whole
+  // 64-byte (act) or 128-byte (routed) pieces of its rows: straight from the
+  // accumulators (16-byte pieces of 32 rows) the stores took 45 of the down
+  // projection's 150 us at T = 4096.
+  uint8_t *const scratch = const_cast<uint8_t *>(buf);
+  if (KIND == 0) {
+    if (un.nt * (kBN / 2) + w * 32 >= a.I) return slot;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      uint8_t *const sc = scratch + (b & 1 ? a1 : a0);  // 32 rows of 64 bytes
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 8 * c + 2 * j;
+          const uint32_t g = pack_bf16x2(acc[0][b][i], acc[0][b][i + 1]);
+          const uint32_t u = pack_bf16x2(acc[1][b][i], acc[1][b][i + 1]);
+          o[j] = pack_bf16x2(swiglu(bf16_bits_to_f32(g & 0xffffu), bf16_bits_to_f32(u & 0xffffu)),
+                             swiglu(bf16_bits_to_f32(g >> 16), bf16_bits_to_f32(u >> 16)));
+        }
+        *(u32x4 *)(sc + r * 64 + (((2 * h + c) ^ ((r >> 2) & 3)) << 4)) = o;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 16 * i + (lane >> 2), c = lane & 3;
+        const u32x4 o = *(const u32x4 *)(sc + row * 64 + ((c ^ ((row >> 2) & 3)) << 4));
+        if (32 * b + row < un.rows)
+          store_row(a.act + (size_t)(un.row0 + 32 * b + row) * a.I + un.nt * (kBN / 2) + w * 32 + c * 8, o);
+      }
+    }
+  } else {
+    const int col = un.nt * kBN + w * 64 + (lane & 7) * 8;
+    const bool live = un.nt * kBN + w * 64 + (lane & 4) * 8 < a.H;  // 32-column fragments
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      uint8_t *const sc = scratch + (b & 1 ? a1 : a0);  // 32 rows of 128 bytes
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          u32x4 o;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(acc[q][b][8 * c + 2 * j], acc[q][b][8 * c + 2 * j + 1]);
+          *(u32x4 *)(sc + r * 128 + (((4 * q + 2 * h + c) ^ ((r >> 1) & 7)) << 4)) = o;
+        }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        const u32x4 o = *(const u32x4 *)(sc + row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+        const int q0 = __shfl(route[b], row, kWave);
+        if (q0 >= 0 && live) store_row(a.routed + (size_t)q0 * a.H + col, o);
+      }
+    }
+  }
+  return slot;
+}
+
+template <int KIND, int NBM>
+__global__ __launch_bounds__(kThreads) void tile_kernel(ExpertArgs a, int max_rows) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int wave = sgpr(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tasks = *as_const(a.num_tasks);
+  UnitMap map;
+  map.init(a.counts, a.offsets, a.E, KIND == 0 ? (a.I + kBN / 2 - 1) / (kBN / 2) : (a.H + kBN - 1) / kBN, max_rows,
+           lane);
+  if (tasks == 0) return;  // no route, or a plan that stalled
+  // One contiguous chunk of the unit sequence per XCD (consecutive workgroup
+  // IDs go round-robin over the XCDs), walked by the XCD's workgroups together.
+  const int G = gridDim.x;
+  const bool xcd_mode = G % 8 == 0;
+  const int P = xcd_mode ? G / 8 : G;  // workgroups per chunk
+  const int xcd = xcd_mode ? (int)blockIdx.x % 8 : 0;
+  const int p = xcd_mode ? (int)blockIdx.x / 8 : (int)blockIdx.x;
+  const int CH = xcd_mode ? (map.total + 7) / 8 : map.total;  // units per chunk
+  const int c_end = min(CH, map.total - xcd * CH);
+  const int nu = p < c_end ? (c_end - p + P - 1) / P : 0;
+  const int first = xcd * CH + p;
+  if (wave >= kMfmaWaves) {
+    load_role<KIND, NBM>(a, map, first, P, nu, wave - kMfmaWaves, lane, smem);
+    return;
+  }
+  const int KT = ((KIND == 0 ? a.H : a.I) + kBK - 1) / kBK;
+  int slot = 0;
+  for (int i = 0; i < nu; ++i) {
+    const UnitMap::Unit un = map.at(first + i * P);
+    slot = sgpr(slot);
+    const int nb = sgpr((un.rows + 31) >> 5);
+    if (nb == 1) {
+      slot = mfma_unit<KIND, 1, NBM>(a, un, KT, slot, wave, lane, smem);
+    } else if (NBM == 2 || nb == 2) {
+      slot = mfma_unit<KIND, 2, NBM>(a, un, KT, slot, wave, lane, smem);
+    } else if constexpr (NBM > 2) {
+      if (nb == 3) slot = mfma_unit<KIND, 3, NBM>(a, un, KT, slot, wave, lane, smem);
+      else if (nb == 4) slot = mfma_unit<KIND, 4, NBM>(a, un, KT, slot, wave, lane, smem);
+      else slot = mfma_unit<KIND, 5, NBM>(a, un, KT, slot, wave, lane, smem);
     }
   }
 }
 
-template <int KIND>
-hipError_t launch_tile_ws(const ExpertArgs &a, int units_bound, int num_cus, hipStream_t s) {
-  using C = TileCfg<KIND>;
-  auto k = tile_ws_kernel<KIND>;
-  const size_t lds = (size_t)kWsStages * C::STAGE_BYTES;
+template <int KIND, int NBM>
+hipError_t launch_nbm(const ExpertArgs &a, int max_rows, int num_cus, hipStream_t s) {
+  auto k = tile_kernel<KIND, NBM>;
+  const size_t lds = (size_t)ring_slots(NBM) * slot_bytes(NBM);
   static bool attr = [&] {
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds) == hipSuccess;
   }();
   if (!attr) return hipErrorInvalidValue;
-  int grid = num_cus;
-  if (grid > units_bound) grid = units_bound;
-  if (grid < 1) grid = 1;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(kWsThreads), lds, s, a);
+  hipLaunchKernelGGL(k, dim3(num_cus), dim3(kThreads), lds, s, a, max_rows);
   return hipGetLastError();
+}
+
+// Token blocks per unit at most, from the shape alone (a captured launch stays
+// valid for any routes).  High units load each weight tile least often and win
+// where experts have many rows: 160-row units against 96-row ones took 307 vs
+// 334 us per layer at E = 128, H = 2048, I = 768, K = 8, T = 2048 (mean 128)
+// and 425 vs 448 at E = 32, H = I = 2880, K = 4, T = 1024 (Zipf routing).
+// Below a mean of 128 rows 96-row units waste less of the last round: T = 1024
+// Zipf 242 vs 255 us, uniform 266 vs 267 (64-row units: 262 and 293).  While
+// the units leave half the CUs idle, lower ones: the four-slot ring of 64 rows
+// (16 experts of 64 rows: 66.3 vs 67.9 us), then 32-row units where an
+// expert's rows still make more of them (E = 8, H = 512, I = 256, 256 rows
+// each: 26.5 vs 28.3 us).
+int unit_blocks(long long R, int E, int ntiles, int num_cus) {
+  const long long mean = (R + E - 1) / E;
+  auto units = [&](int nb) { return (long long)E * ntiles * ((mean + 32 * nb - 1) / (32 * nb)); };
+  int nb = mean >= 128 ? kMaxNB : mean > 40 ? 3 : 2;
+  if (nb == 3 && mean <= 64 && 2 * units(2) <= num_cus) nb = 2;
+  while (nb > 1 && mean > (nb > 2 ? 32 : 64) * (nb - 1) && 2 * units(nb) < num_cus) --nb;
+  return nb;
+}
+
+template <int KIND>
+hipError_t launch_tile(const ExpertArgs &a, int num_cus, hipStream_t s) {
+  const int ntiles = KIND == 0 ? (a.I + kBN / 2 - 1) / (kBN / 2) : (a.H + kBN - 1) / kBN;
+  const int nb = unit_blocks(a.R, a.E, ntiles, num_cus);
+  return nb <= 2 ? launch_nbm<KIND, 2>(a, 32 * nb, num_cus, s) : launch_nbm<KIND, kMaxNB>(a, 32 * nb, num_cus, s);
 }
 
 }  // namespace
 
+bool tile_gemm_ok(int H, int I) {
+  // Whole 32-row fragments and 16-byte chunks; byte offsets within one
+  // expert's matrix, overshoot of the last tile included, fit 32 bits.
+  return H % 32 == 0 && I % 32 == 0 && (long long)H * I * 2 < (1LL << 31);
+}
+
 bool tile_shape_ok(int H, int I, bool w4) {
-  // down (both formats): K = I in 64-wide stages (even count), H in 256-row tiles.
-  if (I % 128 || H % 256) return false;
-  // gate/up: bf16 here, K = H in 64-wide stages (even count), act columns in
-  // 128-column tiles; W4 in the wave kernel.
-  return w4 ? wave_w4_shape_ok(H, I, 64) : H % 128 == 0;
+  if (I % 128 || H % 256 || !tile_gemm_ok(H, I)) return false;
+  return w4 ? wave_w4_shape_ok(H, I, 64) : true;  // W4 gate/up runs in the wave kernel
 }
 
-hipError_t launch_tile_gate_up(const ExpertArgs &a, int task_capacity, int num_cus, hipStream_t s) {
-  return launch_tile_ws<0>(a, task_capacity * (a.I / 128), num_cus, s);
+hipError_t launch_tile_gate_up(const ExpertArgs &a, int num_cus, hipStream_t s) {
+  return launch_tile<0>(a, num_cus, s);
 }
 
-hipError_t launch_tile_down(const ExpertArgs &a, int task_capacity, int num_cus, hipStream_t s) {
-  return launch_tile_ws<1>(a, task_capacity * (a.H / 256), num_cus, s);
+hipError_t launch_tile_down(const ExpertArgs &a, int num_cus, hipStream_t s) {
+  return launch_tile<1>(a, num_cus, s);
 }
 
 }  // namespace moe

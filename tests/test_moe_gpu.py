@@ -120,6 +120,36 @@ def _ids_with_counts(counts, tokens, k):
     return flat.view(k, tokens).t().contiguous().to(torch.int32)
 
 
+@pytest.mark.parametrize("hidden,inter,special", [
+    (2048, 768, [160, 161, 320, 321, 1, 31, 33, 159]),  # units of 96 rows (gate/up) and 160 (down), whole tiles
+    (2080, 800, [128, 129, 64, 65, 97, 32, 480, 2]),    # half stages at the end of K, partial weight tiles
+    (1056, 96, [300, 1, 0, 0, 161, 0, 96, 5]),          # I below one weight tile and one and a half stages
+    (512, 256, [40, 33, 64, 32, 1, 0, 31, 48]),         # 32-row units, four ring slots
+])
+def test_tiled_row_blocks(hidden, inter, special, gpu_device):
+    """The LDS-tiled kernels cut each expert's rows into equal blocks of at most
+    160, 96, 64 or 32: row counts around those edges (and experts without rows),
+    weight tiles and K stages that end inside the matrices.  Each grouped row
+    is checked against the FP32 oracle, and a second run is bitwise equal."""
+    tokens, k, e = 512, 4, 16
+    rest = tokens * k - sum(special)
+    counts = special + [rest // 8 + (1 if i < rest % 8 else 0) for i in range(8)]
+    ids = _ids_with_counts(counts, tokens, k)
+    x, gu, dn, _, _ = O.make_inputs(tokens=tokens, experts=e, topk=k, hidden=hidden, intermediate=inter,
+                                    id_dtype=torch.int32, pattern="random", seed=hidden + inter)
+    w = torch.softmax(torch.randn(tokens, k, generator=torch.Generator().manual_seed(3)), dim=-1)
+    dev = _to(gpu_device, x, gu, dn, ids, w)
+    plan = prepare_moe(*dev, config=GemmConfig(block_m=64))
+    first = plan.run().clone()
+    out = plan.run()
+    torch.cuda.synchronize()
+    plan.check_inputs()
+    assert plan.base.counts.cpu().tolist() == counts
+    assert torch.equal(first.view(torch.int16), out.view(torch.int16))
+    m = O.error(out, O.moe_reference(x, gu, dn, ids.long(), w))
+    assert m["passed"], m
+
+
 def test_w4_pair_passes_at_task_boundaries(gpu_device):
     """W4 gate/up with 64-row tasks (the pair kernel): experts with 1, 33, 64, 65, 96,
     97, 129 and 160 rows cover a single short task, a full task, two tasks run as one
