@@ -162,6 +162,17 @@ constexpr bool kDmaDown = true;
 // products (H = 96, I = 32: 19.5 against 17.2 us).
 static bool generic_tiled(int H, int I) { return tile_gemm_ok(H, I) && (long long)H * I >= 65536; }
 
+// W4 gate/up of 64-row tasks at H = 2048: the register-streaming pair kernel
+// decodes each weight once per 96 rows, the tiled kernel once per 160 and with
+// the MFMA waves free of it.  Measured, pair against tiled (E = 128, I = 768,
+// K = 8): T = 600 88 / 91 us, T = 1024 112 / 114, T = 1536 136 / 143 (Zipf 156 /
+// 150), T = 2048 179 / 143, T = 4096 311 / 233; with few experts the pair
+// kernel's workgroups (16 column blocks of one task) do not fill the CUs: E =
+// 16, 64 rows each 41 / 30 us.
+static bool w4_pair_preferred(const ExpertArgs &a, int num_cus) {
+  return a.H == 2048 && (long long)a.R < 128LL * a.E && (long long)a.E * ((a.I + 255) / 256) * 4 >= num_cus;
+}
+
 hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_block, bool w4,
                           int path, int num_cus, hipStream_t s) {
   // W4 with several rows per expert, and every 64-row task: decode each weight
@@ -169,10 +180,12 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   // row per expert the split-K streaming kernel overlaps the decode better, and
   // with the folded decode it is faster for 16-row tasks too (T = 193: gate/up
   // 49 vs 61 us).
-  const bool wave_ok = w4 && wave_w4_shape_ok(a.H, a.I, token_block);
+  if (w4 && token_block == 64 && !w4_pair_preferred(a, num_cus) && (path == kTile || generic_tiled(a.H, a.I)))
+    return launch_tile_gate_up(a, true, num_cus, s);
+  const bool wave_ok = w4 && (token_block != 64 || a.H == 2048) && wave_w4_shape_ok(a.H, a.I, token_block);
   if (wave_ok && path != kGeneric && (token_block == 64 || ((long long)a.R >= 4LL * a.E && !a.w4_fold)))
     return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (path == kTile) return w4 ? hipErrorInvalidValue : launch_tile_gate_up(a, num_cus, s);
+  if (path == kTile) return w4 ? hipErrorInvalidValue : launch_tile_gate_up(a, false, num_cus, s);
   if (path == kStream) {
     if (!w4 && kDmaStreaming && dma_shape_ok(a.H, a.I, token_block))
       return launch_dma_gate_up(a, token_block, num_cus, s);
@@ -183,7 +196,7 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   // 32) the scalar one.
   if (wave_ok) return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
   if (path == kGeneric && token_block == 64 && !w4 && generic_tiled(a.H, a.I))
-    return launch_tile_gate_up(a, num_cus, s);
+    return launch_tile_gate_up(a, false, num_cus, s);
   if (path == kGeneric && flex_shape_ok(a.H, a.I, w4))
     return launch_flex_gate_up(a, task_capacity, token_block, w4, s);
   if (w4) return hipErrorInvalidValue;

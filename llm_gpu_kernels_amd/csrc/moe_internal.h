@@ -91,8 +91,9 @@ hipError_t launch_dma_gate_up_planned(const ExpertArgs &a, const RouteArgs &ra, 
 bool wave_w4_shape_ok(int H, int I, int token_block);
 hipError_t launch_wave_w4_gate_up(const ExpertArgs &a, int task_capacity, int token_block,
                                   hipStream_t s);
-// LDS-tiled bf16 GEMMs for many rows per expert (64-row tasks), moe_tile.hip.
-hipError_t launch_tile_gate_up(const ExpertArgs &a, int num_cus, hipStream_t s);
+// LDS-tiled bf16 GEMMs for many rows per expert (64-row tasks), moe_tile.hip
+// (W4G128 gate/up too where H % 128 == 0).
+hipError_t launch_tile_gate_up(const ExpertArgs &a, bool w4, int num_cus, hipStream_t s);
 hipError_t launch_tile_down(const ExpertArgs &a, int num_cus, hipStream_t s);
 bool tile_gemm_ok(int H, int I);
 // Shapes that report the tiled family (moe_layout.fast_path 2).

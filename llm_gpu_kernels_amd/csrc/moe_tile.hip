@@ -17,11 +17,13 @@
 // MFMA operand reads are bank-conflict free).  The descriptors are bounded at
 // the expert's matrix: weight rows past I or H, and the chunks of the last
 // stage past K, read as zero, so any H and I that are multiples of 32 run
-// here.  (W4G128 gate/up with many rows per expert runs in the wave kernel of
-// moe_wave.hip; the down weights are bf16 in both formats.)
+// here.  (W4G128 gate/up: load_role_w4 below; the down weights are bf16 in both
+// formats.)
 //
 // Epilogues match the streaming kernels: gate/up round to bf16, SwiGLU in
 // fp32, bf16 act rows; down rounds to bf16 and scatters rows to route order.
+#include <type_traits>
+
 #include "common.h"
 #include "moe_internal.h"
 
@@ -76,6 +78,21 @@ constexpr int kMfmaWaves = 4;
 constexpr int kLoaders = 4;
 constexpr int kThreads = (kMfmaWaves + kLoaders) * kWave;
 constexpr int kAPer = kBN / kLoaders / 8;  // weight loads per loader wave and stage
+// Where stage buffers sit in the LDS.  bf16: each slot holds a weight tile and a
+// token tile.  W4: two weight tiles (written by the loaders during the stage
+// before they are read) and, in what is left, as many token tiles as fit up
+// to eight, so that their loads are three stages ahead or more.
+template <int NBM, bool W4>
+struct Ring {
+  static constexpr int kBBytes = NBM * 32 * kBK * 2;
+  static constexpr int kASlots = W4 ? 2 : ring_slots(NBM);
+  static constexpr int kBFit = (kRingBytes - 2 * kABytes) / kBBytes;
+  static constexpr int kBSlots = W4 ? (kBFit < 8 ? kBFit : 8) : ring_slots(NBM);
+  static constexpr int kAStride = W4 ? kABytes : slot_bytes(NBM);
+  static constexpr int kB0 = W4 ? 2 * kABytes : kABytes;
+  static constexpr int kBStride = W4 ? kBBytes : slot_bytes(NBM);
+  static constexpr int kBytes = W4 ? kB0 + kBSlots * kBBytes : kASlots * kAStride;
+};
 static_assert(ring_slots(2) == 4 && ring_slots(kMaxNB) == 3, "the loaders' wait counts cover three and four slots");
 
 // s_waitcnt with only the vector-memory counter bounded (gfx9 encoding).
@@ -187,10 +204,45 @@ __device__ __forceinline__ float swiglu(float g, float u) {
 // end of the kernel, when nothing else runs (down at T = 1024: 87 -> 79 us).
 __device__ __forceinline__ void store_row(uint16_t *p, u32x4 v) { __builtin_nontemporal_store(v, (u32x4 *)p); }
 
+// 16-byte chunk c of row m of a stage's 32-row fragment sits at chunk c ^
+// swz(m): the sixteen lanes of an operand read (consecutive rows, one chunk)
+// and of the W4 loaders' writes (rows 8 q + 4 hb + i, one chunk) each cover all
+// 64 banks.
+__device__ __forceinline__ int swz(int m) { return ((m >> 1) & 7) ^ ((m >> 3) & 2); }
+
 // Weight row within a 32-row fragment that LDS row m of it holds: the MFMA
 // leaves output rows 8 q + 4 h + i (q, i = 0..3) in lane half h, so with this
 // order a lane's sixteen outputs are sixteen consecutive columns.
 __device__ __forceinline__ int frag_row(int m) { return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3); }
+
+// Token of this lane's row 32 b + 8 lw + lr of each token block of a unit, rows
+// past the unit's end repeating its first row.  Scalar loads, every one of
+// them issued before the first is used and none behind a branch: the
+// vector-memory counter holds only LDS loads, so nothing here waits on those,
+// and the loaders stand still for one memory round trip per unit (with the
+// loads behind per-row conditions, up to forty in a row, T = 4096 gate/up took
+// 237 us instead of 232).  Blocks past the unit's rows read block 0's tokens.
+template <int NBM>
+__device__ __forceinline__ void token_rows(const ExpertArgs &a, const UnitMap::Unit &un, int lw, int lr,
+                                           uint32_t (&rows)[NBM]) {
+  const MOE_CONST int32_t *rt = as_const(a.row_token) + un.row0;
+  const int nb = (un.rows + 31) >> 5;
+  const int t0 = rt[0];
+  int tk[NBM][8];
+#pragma unroll
+  for (int b = 0; b < NBM; ++b) {
+    const MOE_CONST int32_t *p = rt + (b < nb ? b : 0) * 32 + lw * 8;  // at most 31 rows past the unit's end
+#pragma unroll
+    for (int k = 0; k < 8; ++k) tk[b][k] = p[k];
+  }
+#pragma unroll
+  for (int b = 0; b < NBM; ++b) {
+    int tok = tk[b][0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) tok = lr == k ? tk[b][k] : tok;
+    rows[b] = (uint32_t)(b * 32 + lw * 8 + lr < un.rows ? tok : t0);
+  }
+}
 
 template <int KIND, int NBM>
 __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &map, int first, int stride, int nu,
@@ -206,14 +258,14 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
 
   // Loader wave lw moves LDS rows [64 lw, +64) of the weight tile and rows
   // 32 b + 8 lw .. + 8 of each token block, eight rows (1 KiB) per load.  LDS
-  // chunk lane % 8 of row r holds logical chunk (lane % 8) ^ ((r >> 1) & 7).
+  // chunk lane % 8 of row r holds logical chunk (lane % 8) ^ swz(r).
   const uint8_t *xbase = KIND == 0 ? (const uint8_t *)a.x : (const uint8_t *)a.act;
   const uint32_t xbytes = KIND == 0 ? (uint32_t)a.T * pitch : (uint32_t)a.R * pitch;
   const auto brs = __builtin_amdgcn_make_buffer_rsrc((void *)xbase, (short)0, (int)xbytes, 0x00020000);
   __amdgpu_buffer_rsrc_t ars;
   uint32_t aoff[kAPer], boff[NBM];
-  // Rows r = 8 j + lr with j even or odd: (r >> 1) & 7 = 4 (j & 1) + lr / 2.
-  const uint32_t c0 = (uint32_t)((lane & 7) ^ (lr >> 1));  // j even; odd: ^ 4
+  // Rows r = 8 j + lr: swz(r) = (lr / 2) ^ 4 (j & 1) ^ (j & 2).
+  const uint32_t c0 = (uint32_t)((lane & 7) ^ (lr >> 1));
   int cur = -1, nb = 0;
   auto setup = [&](int i) {
     const UnitMap::Unit un = map.at(first + i * stride);
@@ -227,30 +279,15 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
 #pragma unroll
     for (int j = 0; j < kAPer; ++j) {
       const int row = wrow0 + (j / 4) * 32 + frag_row((j & 3) * 8 + lr);
-      aoff[j] = (uint32_t)row * pitch + ((c0 ^ (4u * (j & 1))) << 4);
+      aoff[j] = (uint32_t)row * pitch + ((c0 ^ (4u * (j & 1)) ^ (j & 2u)) << 4);
     }
-    // Token of each row through scalar loads (the vector-memory counter holds
-    // only LDS loads, so nothing here waits on them); rows past the unit's
-    // end repeat its first row.
-    const MOE_CONST int32_t *rt = as_const(a.row_token) + un.row0;
+    uint32_t rows[NBM];
+    if (KIND == 0) token_rows<NBM>(a, un, lw, lr, rows);
 #pragma unroll
     for (int b = 0; b < NBM; ++b) {
-      if (b >= nb) break;
-      const int r0 = b * 32 + lw * 8;
-      uint32_t off;
-      if (KIND == 0) {
-        const int t0 = rt[0];
-        int tok = t0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int tk = r0 + k < un.rows ? rt[r0 + k] : t0;
-          tok = lr == k ? tk : tok;
-        }
-        off = (uint32_t)tok * pitch;
-      } else {
-        off = (uint32_t)(un.row0 + (r0 + lr < un.rows ? r0 + lr : 0)) * pitch;
-      }
-      boff[b] = off + ((c0 ^ (4u * (lw & 1))) << 4);
+      const int r0 = b * 32 + lw * 8 + lr;
+      if (KIND == 1) rows[b] = (uint32_t)(un.row0 + (r0 < un.rows ? r0 : 0));
+      boff[b] = rows[b] * pitch + ((c0 ^ (4u * (lw & 1)) ^ (lw & 2u)) << 4);
     }
   };
   int slot = 0, kt_next = 0, unit_next = 0;
@@ -264,7 +301,7 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
     const uint32_t koff = (uint32_t)kt_next * (kBK * 2);
     const bool part = tail != 0 && kt_next == KT - 1;
     const uint32_t oe = part && c0 >= tail ? 0xffffffffu : 0u;         // chunks past K: out of range
-    const uint32_t oo = part && (c0 ^ 4u) >= tail ? 0xffffffffu : 0u;
+    const uint32_t oo = part && (c0 ^ 4u) >= tail ? 0xffffffffu : 0u;  // (tail is 4: bit 1 of c plays no part)
 #pragma unroll
     for (int j = 0; j < kAPer; ++j)
       buffer_load_lds16(ars, buf + (lw * 64 + j * 8) * 128, aoff[j] | (j & 1 ? oo : oe), koff);
@@ -299,12 +336,169 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
   }
 }
 
-// One unit on MFMA wave w with NB token blocks; `slot` is the ring slot of the
-// unit's first stage, returned advanced.
-template <int KIND, int NB, int NBM>
-__device__ __forceinline__ int mfma_unit(const ExpertArgs &a, const UnitMap::Unit &un, int KT, int slot, int w,
-                                         int lane, const uint8_t *smem) {
-  constexpr int kSlots = ring_slots(NBM), kSlotBytes = slot_bytes(NBM);
+// 16 bytes of LDS per lane, written from inline assembly: the compiler would
+// make an LDS store of its own wait for every LDS-destination load in flight,
+// here the token tiles of the next stages.  Completed by an explicit
+// lgkmcnt(0) before the stage's barrier.
+template <int OFF>
+__device__ __forceinline__ void lds_write_b128(uint32_t addr, u32x4 v) {
+  asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "i"(OFF) : "memory");
+}
+
+// W4G128 gate/up: the loader waves stream the int4 words into registers (one
+// 1 KiB load per 16 rows x 128 K, i.e. per two stages, three pairs of stages ahead),
+// decode them bit-exactly and write the bf16 weight tile of stage st + 2 while
+// the MFMA waves multiply stage st, so each weight is decoded once per unit of
+// up to 160 rows and the MFMA waves issue no decode.  Token tiles come as in
+// the bf16 kernel, always NBM loads per stage (blocks past the unit's rows are
+// out of range), so every wait is a constant count.  T = 4096, E = 128, H =
+// 2048, I = 768, K = 8: 233 us (885 TFLOP/s) against 311 us with the pair
+// kernel, as fast as the bf16 weights; without the word loads and the decode
+// 203 us, so the MFMAs' rate on real data bounds it.
+template <int NBM>
+__device__ __forceinline__ void load_role_w4(const ExpertArgs &a, const UnitMap &map, int first, int stride, int nu,
+                                             int lw, int lane, uint8_t *smem) {
+  using R = Ring<NBM, true>;
+  constexpr int kLead = R::kBSlots - 1;  // token tiles in flight, in stages
+  constexpr int kWLoads = 8;  // words and scales of the wave's four row blocks, per pair
+  const int H = a.H, I = a.I;
+  const int KP = H / 128, KT = 2 * KP;  // pairs and stages per unit
+  const int nstages = nu * KT;
+  if (nstages == 0) return;
+  const uint32_t pitch = (uint32_t)H * 2u;
+  const int r = lane & 15, g = lane >> 4;
+
+  // ---- token tiles ----
+  const auto brs = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, (int)((uint32_t)a.T * pitch), 0x00020000);
+  const int lr = lane >> 3;
+  const uint32_t bchunk = (uint32_t)((lane & 7) ^ swz(8 * lw + lr)) << 4;
+  uint32_t boff[NBM];
+  int b_unit = 0, b_kt = 0, b_slot = 0;
+  auto issue_b = [&]() __attribute__((always_inline)) {
+    if (b_kt == 0) {
+      const bool in = b_unit < nu;  // past the last unit: loads that read nothing
+      const UnitMap::Unit un = map.at(first + (in ? b_unit : nu - 1) * stride);
+      uint32_t rows[NBM];
+      token_rows<NBM>(a, un, lw, lr, rows);
+#pragma unroll
+      for (int b = 0; b < NBM; ++b) boff[b] = in && b * 32 < un.rows ? rows[b] * pitch + bchunk : 0xffffffffu;
+    }
+    uint8_t *dst = smem + R::kB0 + b_slot * R::kBStride + lw * 8 * 128;
+#pragma unroll
+    for (int b = 0; b < NBM; ++b) buffer_load_lds16(brs, dst + b * 32 * 128, boff[b], (uint32_t)b_kt * (kBK * 2));
+    b_slot = b_slot == R::kBSlots - 1 ? 0 : b_slot + 1;
+    if (++b_kt == KT) {
+      b_kt = 0;
+      ++b_unit;
+    }
+  };
+
+  // ---- weight words: blocks f, hb = rows 32 f + 16 hb .. + 16 of the wave's 64 ----
+  u32x4 wq[3][4];
+  uint32_t sc[3][4];
+  const uint32_t half_words = (uint32_t)I * (uint32_t)H / 2u, half_scales = (uint32_t)(I / 16) * KP * 32u;
+  __amdgpu_buffer_rsrc_t wrs, srs;
+  uint32_t woff = 0, soff = 0;
+  int w_unit = 0, w_kp = 0;
+  auto issue_w = [&](int buf) __attribute__((always_inline)) {
+    if (w_kp == 0) {
+      const UnitMap::Unit un = map.at(first + min(w_unit, nu - 1) * stride);
+      const size_t half = (size_t)un.e * 2 + (lw >> 1);  // gate rows, then up rows
+      wrs = __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)a.w4_words + half * half_words), (short)0,
+                                              (int)half_words, 0x00020000);
+      srs = __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)a.w4_scales + half * half_scales), (short)0,
+                                              (int)half_scales, 0x00020000);
+      const uint32_t n16 = (uint32_t)(un.nt * (kBN / 2) + (lw & 1) * 64) / 16u;
+      woff = n16 * (uint32_t)KP * 1024u + (uint32_t)lane * 16u;
+      soff = n16 * (uint32_t)KP * 32u + (uint32_t)r * 2u;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      wq[buf][j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, woff + (uint32_t)(j * KP) * 1024u, w_kp * 1024, 0));
+      sc[buf][j] = __builtin_amdgcn_raw_buffer_load_b16(srs, soff + (uint32_t)(j * KP) * 32u, w_kp * 32, 0);
+    }
+    if (++w_kp == KP) {
+      w_kp = 0;
+      ++w_unit;
+    }
+  };
+  // Weight row 16 hb + r of a fragment sits in LDS row m = 8 (r / 4) + 4 hb +
+  // r % 4 (frag_row's inverse); word 2 s + jj of a lane is chunk 4 jj + g of
+  // stage half s.
+  uint32_t wdst[2][2];
+#pragma unroll
+  for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const int m = 8 * (r >> 2) + 4 * hb + (r & 3);
+      wdst[hb][jj] = (uint32_t)(lw * 64 + m) * 128u + (((4 * jj + g) ^ swz(m)) << 4) +
+                     (uint32_t)(uintptr_t)(const MOE_LDS uint8_t *)smem;
+    }
+  int d_slot = 0;
+  auto decode = [&](int buf, int s) __attribute__((always_inline)) {
+    const uint32_t base = (uint32_t)(d_slot * R::kAStride);
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        const W4Scale k = w4_scale(bf16_bits_to_f32(sc[buf][2 * f + hb]));
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+          const u32x4 v = w4_decode8(wq[buf][2 * f + hb][2 * s + jj], k);
+          if (f == 0) lds_write_b128<0>(base + wdst[hb][jj], v);
+          else lds_write_b128<4096>(base + wdst[hb][jj], v);
+        }
+      }
+    d_slot ^= 1;
+  };
+
+#pragma unroll
+  for (int i = 0; i < kLead; ++i) issue_b();
+  issue_w(0);
+  issue_w(1);
+  issue_w(2);
+  decode(0, 0);
+  int st = 0;
+  // Stage st is published, stage st + 1 decoded (half 1 of a pair in even
+  // stages) and the token tile of stage st + kLead requested.  The token tile
+  // of stage st was followed by kLead - 1 later ones and by the words issued
+  // in the even ones of stages st - kLead .. st - 1.
+  auto stage = [&](auto even, int buf) __attribute__((always_inline)) {
+    constexpr int kWords = decltype(even)::value ? kLead / 2 : (kLead + 1) / 2;
+    constexpr int kLater = (kLead - 1) * NBM + kWords * kWLoads;
+    constexpr int kWait = kLater < 63 ? kLater : 63;
+    __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue_b();
+    if (st + 1 < nstages) decode(buf, decltype(even)::value ? 1 : 0);
+    if (decltype(even)::value) issue_w(buf);  // the pair three after the one just decoded
+    ++st;
+  };
+  const std::true_type even;
+  const std::false_type odd;
+  while (true) {  // nstages is even; word buffers 0, 1, 2 in turn
+    stage(even, 0);
+    stage(odd, 1);
+    if (st >= nstages) break;
+    stage(even, 1);
+    stage(odd, 2);
+    if (st >= nstages) break;
+    stage(even, 2);
+    stage(odd, 0);
+    if (st >= nstages) break;
+  }
+  wait_vmcnt<0>();  // nothing may reach the LDS after the workgroup has ended
+}
+
+// One unit on MFMA wave w with NB token blocks; a_slot and b_slot are the ring
+// slots of the unit's first stage, advanced past its last.
+template <int KIND, int NB, int NBM, bool W4>
+__device__ __forceinline__ void mfma_unit(const ExpertArgs &a, const UnitMap::Unit &un, int KT, int &a_slot,
+                                          int &b_slot, int w, int lane, const uint8_t *smem) {
+  using R = Ring<NBM, W4>;
   const int r = lane & 31, h = lane >> 5;
   f32x16 acc[2][NB];
 #pragma unroll
@@ -323,45 +517,47 @@ __device__ __forceinline__ int mfma_unit(const ExpertArgs &a, const UnitMap::Uni
   // Byte offset of this lane's chunk of K-step ks within a 32-row fragment.
   uint32_t lo[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) lo[ks] = (uint32_t)(r * 128 + (((2 * ks + h) ^ ((r >> 1) & 7)) << 4));
+  for (int ks = 0; ks < 4; ++ks) lo[ks] = (uint32_t)(r * 128 + (((2 * ks + h) ^ swz(r)) << 4));
   const uint32_t a0 = KIND == 0 ? w * 4096 : w * 8192, a1 = KIND == 0 ? 16384 + w * 4096 : w * 8192 + 4096;
 
   // One K-step: the MFMAs of the fragments read a step ago, with the next
   // step's fragment reads issued between them.
   u32x4 af[2][2], bf[2][NB];
-  auto read_one = [&](int set, const uint8_t *buf, int ks, int i) __attribute__((always_inline)) {
-    if (i == 0) af[set][0] = *(const u32x4 *)(buf + a0 + lo[ks]);
-    else if (i == 1) bf[set][0] = *(const u32x4 *)(buf + kABytes + lo[ks]);
-    else if (i == 2) af[set][1] = *(const u32x4 *)(buf + a1 + lo[ks]);
-    else if (i < NB + 2) bf[set][i - 2] = *(const u32x4 *)(buf + kABytes + (i - 2) * 4096 + lo[ks]);
+  const uint8_t *abuf = smem, *bbuf = smem;
+  auto read_one = [&](int set, int ks, int i) __attribute__((always_inline)) {
+    if (i == 0) af[set][0] = *(const u32x4 *)(abuf + a0 + lo[ks]);
+    else if (i == 1) bf[set][0] = *(const u32x4 *)(bbuf + lo[ks]);
+    else if (i == 2) af[set][1] = *(const u32x4 *)(abuf + a1 + lo[ks]);
+    else if (i < NB + 2) bf[set][i - 2] = *(const u32x4 *)(bbuf + (i - 2) * 4096 + lo[ks]);
   };
-  auto read_all = [&](int set, const uint8_t *buf, int ks) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NB + 2; ++i) read_one(set, buf, ks, i);
-  };
-  auto step = [&](int set, const uint8_t *buf, int ks) __attribute__((always_inline)) {
+  auto step = [&](int set, int ks) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 2 * NB; ++i) {
       acc[i & 1][i >> 1] = mfma32(af[set][i & 1], bf[set][i >> 1], acc[i & 1][i >> 1]);
       if (i < NB + 2) {
         __builtin_amdgcn_sched_barrier(0);
-        read_one(set ^ 1, buf, ks, i);
+        read_one(set ^ 1, ks, i);
         if (i == 2 * NB - 1)
-          for (int j = 2 * NB; j < NB + 2; ++j) read_one(set ^ 1, buf, ks, j);
+          for (int j = 2 * NB; j < NB + 2; ++j) read_one(set ^ 1, ks, j);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  const uint8_t *buf = smem;
   for (int kt = 0; kt < KT; ++kt) {
     lds_barrier();  // the stage is published; every read of the stage before it is done
-    buf = smem + slot * kSlotBytes;
-    slot = slot == kSlots - 1 ? 0 : slot + 1;
-    if (kt == 0) read_all(0, buf, 0);
-    else step(1, buf, 0);
-    step(0, buf, 1);
-    step(1, buf, 2);
-    step(0, buf, 3);
+    abuf = smem + a_slot * R::kAStride;
+    bbuf = smem + R::kB0 + b_slot * R::kBStride;
+    a_slot = a_slot == R::kASlots - 1 ? 0 : a_slot + 1;
+    b_slot = b_slot == R::kBSlots - 1 ? 0 : b_slot + 1;
+    if (kt == 0) {
+#pragma unroll
+      for (int i = 0; i < NB + 2; ++i) read_one(0, 0, i);
+    } else {
+      step(1, 0);
+    }
+    step(0, 1);
+    step(1, 2);
+    step(0, 3);
   }
 #pragma unroll
   for (int i = 0; i < 2 * NB; ++i) acc[i & 1][i >> 1] = mfma32(af[1][i & 1], bf[1][i >> 1], acc[i & 1][i >> 1]);
@@ -373,9 +569,9 @@ __device__ __forceinline__ int mfma_unit(const ExpertArgs &a, const UnitMap::Uni
   // 64-byte (act) or 128-byte (routed) pieces of its rows: straight from the
   // accumulators (16-byte pieces of 32 rows) the stores took 45 of the down
   // projection's 150 us at T = 4096.
-  uint8_t *const scratch = const_cast<uint8_t *>(buf);
+  uint8_t *const scratch = const_cast<uint8_t *>(abuf);
   if (KIND == 0) {
-    if (un.nt * (kBN / 2) + w * 32 >= a.I) return slot;
+    if (un.nt * (kBN / 2) + w * 32 >= a.I) return;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       uint8_t *const sc = scratch + (b & 1 ? a1 : a0);  // 32 rows of 64 bytes
@@ -424,10 +620,9 @@ __device__ __forceinline__ int mfma_unit(const ExpertArgs &a, const UnitMap::Uni
       }
     }
   }
-  return slot;
 }
 
-template <int KIND, int NBM>
+template <int KIND, int NBM, bool W4>
 __global__ __launch_bounds__(kThreads) void tile_kernel(ExpertArgs a, int max_rows) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int wave = sgpr(threadIdx.x >> 6);
@@ -449,31 +644,36 @@ __global__ __launch_bounds__(kThreads) void tile_kernel(ExpertArgs a, int max_ro
   const int nu = p < c_end ? (c_end - p + P - 1) / P : 0;
   const int first = xcd * CH + p;
   if (wave >= kMfmaWaves) {
-    load_role<KIND, NBM>(a, map, first, P, nu, wave - kMfmaWaves, lane, smem);
+    if constexpr (W4) load_role_w4<NBM>(a, map, first, P, nu, wave - kMfmaWaves, lane, smem);
+    else load_role<KIND, NBM>(a, map, first, P, nu, wave - kMfmaWaves, lane, smem);
     return;
   }
   const int KT = ((KIND == 0 ? a.H : a.I) + kBK - 1) / kBK;
-  int slot = 0;
+  int sa = 0, sb = 0;
   for (int i = 0; i < nu; ++i) {
     const UnitMap::Unit un = map.at(first + i * P);
-    slot = sgpr(slot);
+    sa = sgpr(sa);
+    sb = sgpr(sb);
     const int nb = sgpr((un.rows + 31) >> 5);
     if (nb == 1) {
-      slot = mfma_unit<KIND, 1, NBM>(a, un, KT, slot, wave, lane, smem);
+      mfma_unit<KIND, 1, NBM, W4>(a, un, KT, sa, sb, wave, lane, smem);
     } else if (NBM == 2 || nb == 2) {
-      slot = mfma_unit<KIND, 2, NBM>(a, un, KT, slot, wave, lane, smem);
+      mfma_unit<KIND, 2, NBM, W4>(a, un, KT, sa, sb, wave, lane, smem);
     } else if constexpr (NBM > 2) {
-      if (nb == 3) slot = mfma_unit<KIND, 3, NBM>(a, un, KT, slot, wave, lane, smem);
-      else if (nb == 4) slot = mfma_unit<KIND, 4, NBM>(a, un, KT, slot, wave, lane, smem);
-      else slot = mfma_unit<KIND, 5, NBM>(a, un, KT, slot, wave, lane, smem);
+      if (NBM == 3 || nb == 3) {
+        mfma_unit<KIND, 3, NBM, W4>(a, un, KT, sa, sb, wave, lane, smem);
+      } else if constexpr (NBM > 3) {
+        if (nb == 4) mfma_unit<KIND, 4, NBM, W4>(a, un, KT, sa, sb, wave, lane, smem);
+        else mfma_unit<KIND, 5, NBM, W4>(a, un, KT, sa, sb, wave, lane, smem);
+      }
     }
   }
 }
 
-template <int KIND, int NBM>
+template <int KIND, int NBM, bool W4>
 hipError_t launch_nbm(const ExpertArgs &a, int max_rows, int num_cus, hipStream_t s) {
-  auto k = tile_kernel<KIND, NBM>;
-  const size_t lds = (size_t)ring_slots(NBM) * slot_bytes(NBM);
+  auto k = tile_kernel<KIND, NBM, W4>;
+  const size_t lds = (size_t)Ring<NBM, W4>::kBytes;
   static bool attr = [&] {
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds) == hipSuccess;
@@ -503,11 +703,14 @@ int unit_blocks(long long R, int E, int ntiles, int num_cus) {
   return nb;
 }
 
-template <int KIND>
+template <int KIND, bool W4>
 hipError_t launch_tile(const ExpertArgs &a, int num_cus, hipStream_t s) {
   const int ntiles = KIND == 0 ? (a.I + kBN / 2 - 1) / (kBN / 2) : (a.H + kBN - 1) / kBN;
   const int nb = unit_blocks(a.R, a.E, ntiles, num_cus);
-  return nb <= 2 ? launch_nbm<KIND, 2>(a, 32 * nb, num_cus, s) : launch_nbm<KIND, kMaxNB>(a, 32 * nb, num_cus, s);
+  if (nb <= 2) return launch_nbm<KIND, 2, W4>(a, 32 * nb, num_cus, s);
+  // W4 loads (and zero-fills) NBM token blocks per stage.
+  if (W4 && nb == 3) return launch_nbm<KIND, W4 ? 3 : kMaxNB, W4>(a, 32 * nb, num_cus, s);
+  return launch_nbm<KIND, kMaxNB, W4>(a, 32 * nb, num_cus, s);
 }
 
 }  // namespace
@@ -523,12 +726,12 @@ bool tile_shape_ok(int H, int I, bool w4) {
   return w4 ? wave_w4_shape_ok(H, I, 64) : true;  // W4 gate/up runs in the wave kernel
 }
 
-hipError_t launch_tile_gate_up(const ExpertArgs &a, int num_cus, hipStream_t s) {
-  return launch_tile<0>(a, num_cus, s);
+hipError_t launch_tile_gate_up(const ExpertArgs &a, bool w4, int num_cus, hipStream_t s) {
+  return w4 ? launch_tile<0, true>(a, num_cus, s) : launch_tile<0, false>(a, num_cus, s);
 }
 
 hipError_t launch_tile_down(const ExpertArgs &a, int num_cus, hipStream_t s) {
-  return launch_tile<1>(a, num_cus, s);
+  return launch_tile<1, false>(a, num_cus, s);
 }
 
 }  // namespace moe

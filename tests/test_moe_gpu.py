@@ -120,13 +120,16 @@ def _ids_with_counts(counts, tokens, k):
     return flat.view(k, tokens).t().contiguous().to(torch.int32)
 
 
-@pytest.mark.parametrize("hidden,inter,special", [
-    (2048, 768, [160, 161, 320, 321, 1, 31, 33, 159]),  # units of 96 rows (gate/up) and 160 (down), whole tiles
-    (2080, 800, [128, 129, 64, 65, 97, 32, 480, 2]),    # half stages at the end of K, partial weight tiles
-    (1056, 96, [300, 1, 0, 0, 161, 0, 96, 5]),          # I below one weight tile and one and a half stages
-    (512, 256, [40, 33, 64, 32, 1, 0, 31, 48]),         # 32-row units, four ring slots
+@pytest.mark.parametrize("hidden,inter,w4,special", [
+    (2048, 768, False, [160, 161, 320, 321, 1, 31, 33, 159]),  # units of 96 rows (gate/up) and 160 (down)
+    (2080, 800, False, [128, 129, 64, 65, 97, 32, 480, 2]),    # half stages at the end of K, partial weight tiles
+    (1056, 96, False, [300, 1, 0, 0, 161, 0, 96, 5]),          # I below one weight tile and one and a half stages
+    (512, 256, False, [40, 33, 64, 32, 1, 0, 31, 48]),         # 32-row units, four ring slots
+    (2048, 768, True, [160, 161, 320, 321, 1, 31, 33, 159]),   # W4: 96-row units
+    (1152, 2080, True, [128, 129, 64, 65, 97, 32, 480, 2]),    # 160-row units, nine word pairs, partial tiles
+    (128, 512, True, [300, 1, 0, 0, 161, 0, 96, 5]),           # 32-row units of one word pair (two stages)
 ])
-def test_tiled_row_blocks(hidden, inter, special, gpu_device):
+def test_tiled_row_blocks(hidden, inter, w4, special, gpu_device):
     """The LDS-tiled kernels cut each expert's rows into equal blocks of at most
     160, 96, 64 or 32: row counts around those edges (and experts without rows),
     weight tiles and K stages that end inside the matrices.  Each grouped row
@@ -138,8 +141,13 @@ def test_tiled_row_blocks(hidden, inter, special, gpu_device):
     x, gu, dn, _, _ = O.make_inputs(tokens=tokens, experts=e, topk=k, hidden=hidden, intermediate=inter,
                                     id_dtype=torch.int32, pattern="random", seed=hidden + inter)
     w = torch.softmax(torch.randn(tokens, k, generator=torch.Generator().manual_seed(3)), dim=-1)
-    dev = _to(gpu_device, x, gu, dn, ids, w)
-    plan = prepare_moe(*dev, config=GemmConfig(block_m=64))
+    xd, dnd, idd, wd = _to(gpu_device, x, dn, ids, w)
+    if w4:
+        packed = quantize_gate_up(gu)
+        plan = prepare_w4_moe(xd, packed, dnd, idd, wd, down_config=GemmConfig(block_m=64))
+        gu = O.dequantize_w4(packed.words, packed.scales)
+    else:
+        plan = prepare_moe(xd, *_to(gpu_device, gu), dnd, idd, wd, config=GemmConfig(block_m=64))
     first = plan.run().clone()
     out = plan.run()
     torch.cuda.synchronize()
