@@ -619,21 +619,58 @@ int gqa_workgroups(int T, int Hkv, int G, int rb) {
 // per CU, four-wave workgroups and no split; otherwise eight-wave
 // workgroups, one per CU, and the keys split half as many times as would fill
 // the CUs (the merge launch and its partial states cost more than idle CUs).
-GqaShape gqa_shape(int T, int Hq, int Hkv, int num_cus) {
+// Key splits of the long-chunk kernel where it is expected to be faster than the
+// shapes below, else 0.  Times in ns, fitted on 256 CUs for T >= 256.  That
+// kernel takes 6 us + 1.43 us per 64-key stage, up to 1.85 with every CU busy
+// (clocks); its workgroups
+// start with the last query blocks, so with R rounds of them the busiest CU
+// runs the first block or R middle ones; a split adds the merge launch and
+// its partial states.  The kernel of this file takes 10 us + 10 ns per token +
+// 1 us per 790 MFLOP.  Measured (T x history, 32 / 8 heads; this file -> long
+// chunk): 2048 x 10816 510 -> 378 us, 2048 x 1792 148 -> 114, 2048 x 17 81 -> 65,
+// 1500 x 4100 168 -> 148, 1024 x 10816 249 -> 202 (two splits), 512 x 10816 134
+// -> 113 (four); 1024 x 1792 68 -> 68, 512 x 1792 32 -> 41, 256 x 4096 35 -> 44.
+int gqa_prefill_splits(int T, int Hq, int Hkv, long long history, int num_cus) {
+  const int wp = gqa_prefill_workgroups(T, Hq, Hkv);
+  if (wp <= 0 || T < 256) return 0;
+  const int nqb = wp / Hkv, qt = 256 / (Hq / Hkv);
+  const double flops = 512.0 * Hq * ((double)T * history + 0.5 * T * (T + 1.0));
+  double best = 0.97 * (10e3 + 10.0 * T + flops / 790e3);
+  int pick = 0;
+  for (int s = 1; s <= kMaxSplits && 64LL * s <= history + T; ++s) {
+    const long long wgs = (long long)wp * s;
+    const long long rounds = (wgs + num_cus - 1) / num_cus;
+    long long mid = num_cus * rounds / 2 / ((long long)Hkv * s);
+    mid = mid < nqb ? mid : nqb - 1;
+    const double longest = (double)(history + T) / 64.0 / s;
+    const double middle = rounds > 1 ? rounds * (double)(history + T - mid * qt) / 64.0 / s : 0.0;
+    const double busy = rounds > 1 ? 1.0 : (double)wgs / num_cus;
+    double t = 6e3 + (longest > middle ? longest : middle) * (1430.0 + 420.0 * busy);
+    if (s > 1) t += 10e3 + (double)T * Hq * s * 1040.0 / 4e3;
+    if (t < best) {
+      best = t;
+      pick = s;
+    }
+  }
+  return pick;
+}
+
+GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus) {
   const int G = Hq / Hkv;
+  if (const int s = gqa_prefill_splits(T, Hq, Hkv, history, num_cus)) return {s, 12, 2, true};
   const int w1 = gqa_workgroups(T, Hkv, G, 1);
-  if (w1 <= 0) return {1, 4, 2};
+  if (w1 <= 0) return {1, 4, 2, false};
   if (w1 <= num_cus) {
-    if (2 * w1 > num_cus) return {1, 8, 1};
+    if (2 * w1 > num_cus) return {1, 8, 1, false};
     const int s = num_cus / w1;
-    return {s < 4 ? s : 4, 4, 1};
+    return {s < 4 ? s : 4, 4, 1, false};
   }
   const int w2 = gqa_workgroups(T, Hkv, G, 2);
-  if (w2 >= 2 * num_cus) return {1, 4, 2};
+  if (w2 >= 2 * num_cus) return {1, 4, 2, false};
   int s = num_cus / w2 / 2;
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;
-  return {s, 8, 2};
+  return {s, 8, 2, false};
 }
 
 size_t gqa_partial_bytes(int T, int Hq, int nsplit) {
@@ -653,24 +690,31 @@ hipError_t launch_fwd(const GqaArgs &a, int hpw, dim3 grid, int groups, int nqb,
   return hipGetLastError();
 }
 
+static hipError_t launch_merge(const GqaArgs &a, int nsplit, hipStream_t s) {
+  hipLaunchKernelGGL(gqa_merge_kernel, dim3((a.T * a.Hq + kMergeRows - 1) / kMergeRows),
+                     dim3(kD * kMergeRows), 0, s, a, nsplit);
+  return hipGetLastError();
+}
+
 hipError_t launch_gqa(const GqaArgs &a, GqaShape shape, hipStream_t s) {
   if (a.T == 0) return hipSuccess;
+  const int nsplit = shape.nsplit;
+  hipError_t e;
+  if (shape.prefill) {
+    e = launch_gqa_prefill(a, nsplit, s);
+    return e != hipSuccess || nsplit == 1 ? e : launch_merge(a, nsplit, s);
+  }
   const int rb = shape.rb, G = a.Hq / a.Hkv, hpw = gqa_heads_per_wg(G, rb);
   const int qt = 16 * (rb / hpw), groups = G / hpw;
   const int nqb = (a.T + qt - 1) / qt;
-  const int nsplit = shape.nsplit;
   const dim3 grid(nqb * a.Hkv * groups * nsplit);
-  hipError_t e;
   if (rb == 1)
     e = shape.waves == 8 ? launch_fwd<1, 8>(a, hpw, grid, groups, nqb, nsplit, s)
                          : launch_fwd<1, 4>(a, hpw, grid, groups, nqb, nsplit, s);
   else
     e = shape.waves == 8 ? launch_fwd<2, 8>(a, hpw, grid, groups, nqb, nsplit, s)
                          : launch_fwd<2, 4>(a, hpw, grid, groups, nqb, nsplit, s);
-  if (e != hipSuccess || nsplit == 1) return e;
-  hipLaunchKernelGGL(gqa_merge_kernel, dim3((a.T * a.Hq + kMergeRows - 1) / kMergeRows),
-                     dim3(kD * kMergeRows), 0, s, a, nsplit);
-  return hipGetLastError();
+  return e != hipSuccess || nsplit == 1 ? e : launch_merge(a, nsplit, s);
 }
 
 }  // namespace moe

@@ -62,7 +62,9 @@ int validate(const gqa_seg_desc *d, int num_cus, moe::GqaShape *shape) {
     return capi_fail(MOE_EINVAL, "q/out must be non-null and 16-byte aligned");
   if ((long long)d->T * d->Hq * 128 >= (1LL << 31))
     return capi_fail(MOE_EINVAL, "T * Hq * 128 must be < 2^31");
-  *shape = moe::gqa_shape(d->T, d->Hq, d->Hkv, num_cus);
+  long long history = 0;
+  for (int s = 0; s + 1 < d->num_segments; ++s) history += d->len[s];
+  *shape = moe::gqa_shape(d->T, d->Hq, d->Hkv, history, num_cus);
   return MOE_OK;
 }
 
@@ -79,7 +81,7 @@ extern "C" {
 
 int gqa_seg_workspace_bytes(const gqa_seg_desc *d, size_t *bytes) {
   int dev = 0, cus = 0;
-  moe::GqaShape shape{1, 4, 2};
+  moe::GqaShape shape{1, 4, 2, false};
   int rc = device_cus(&dev, &cus);
   if (rc) return rc;
   if ((rc = validate(d, cus, &shape))) return rc;
@@ -92,7 +94,7 @@ int gqa_seg_plan_create(gqa_seg_plan **out, const gqa_seg_desc *d) {
   if (!out) return moe::capi_fail(MOE_EINVAL, "null plan pointer");
   *out = nullptr;
   int dev = 0, cus = 0;
-  moe::GqaShape shape{1, 4, 2};
+  moe::GqaShape shape{1, 4, 2, false};
   int rc = device_cus(&dev, &cus);
   if (rc) return rc;
   if ((rc = validate(d, cus, &shape))) return rc;

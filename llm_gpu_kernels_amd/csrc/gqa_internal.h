@@ -23,13 +23,18 @@ struct GqaArgs {
 };
 
 // Launch shape: key splits across workgroups (merged by a second kernel when
-// > 1), waves per workgroup (4 or 8) and 16-row blocks per wave (1 or 2).
+// > 1), waves per workgroup (4 or 8) and 16-row blocks per wave (1 or 2); or
+// the long-chunk kernel (gqa_prefill.hip), whose workgroups share their keys.
 struct GqaShape {
   int nsplit;
   int waves;
   int rb;
+  bool prefill;
 };
-GqaShape gqa_shape(int T, int Hq, int Hkv, int num_cus);
+GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus);
+// Workgroups of the long-chunk kernel before splitting (256 query rows each).
+int gqa_prefill_workgroups(int T, int Hq, int Hkv);
+hipError_t launch_gqa_prefill(const GqaArgs &a, int nsplit, hipStream_t s);
 size_t gqa_partial_bytes(int T, int Hq, int nsplit);
 hipError_t launch_gqa(const GqaArgs &a, GqaShape shape, hipStream_t s);
 

@@ -77,6 +77,27 @@ def test_group_sizes(hq, hkv, gpu_device):
     _check(plan.output, q, segs)
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,history", [
+    (2048, 32, 8, (16, 0, 1)),         # mostly causal, one round of workgroups, no split
+    (530, 32, 8, (8192, 2049, 575)),   # key splits and the merge, ragged last query block
+    (1020, 16, 8, (8000, 100, 3)),     # two heads per KV head
+    (2000, 8, 8, (9000, 0, 65)),       # one head per KV head
+    (700, 64, 8, (6000, 63, 0)),       # eight heads per KV head, an empty segment
+])
+def test_long_chunks(tokens, hq, hkv, history, gpu_device):
+    """The long-chunk kernel (256 query rows per workgroup over shared 64-key
+    stages): every group size, short last tiles of each segment, query blocks
+    that end inside a workgroup, with and without key splits; repeated runs are
+    bitwise equal."""
+    q, segs = _values(tokens, tokens, history, gpu_device, hq=hq, hkv=hkv, v_stride=6144 if tokens == 530 else None)
+    plan = prepare_segmented_gqa(q, segs)
+    first = plan.run().clone()
+    again = plan.run().clone()
+    torch.cuda.synchronize()
+    assert torch.equal(first.view(torch.int16), again.view(torch.int16))
+    _check(first, q, segs)
+
+
 def test_split_merge_partial_workgroup(gpu_device):
     """T * Hq = 66 (query) rows with the keys split: the merge launch's last
     workgroup holds fewer rows than the others."""
