@@ -155,12 +155,42 @@ constexpr bool kDmaDown = true;
 
 }  // namespace
 
-// 64-row tasks of shapes outside the tuned kernels: the LDS-tiled kernels
-// (E = 32, H = I = 2880, T = 512: 312 us per layer against 768 with the
-// run-time-K kernels; E = 128, H = 2048, I = 96, T = 1024: 76 against 113)
-// except for matrices so small that the stage ring's start costs more than the
-// products (H = 96, I = 32: 19.5 against 17.2 us).
-static bool generic_tiled(int H, int I) { return tile_gemm_ok(H, I) && (long long)H * I >= 65536; }
+// Whether a bf16 GEMM runs in the LDS-tiled kernels (`tiles` weight tiles per
+// expert).  The family by shape (path) says so for kTile; beyond it, measured in
+// us per layer unless noted, other kernel against tiled:
+//  * streaming shapes above 16 rows per expert (E = 128, H = 2048, I = 768, K =
+//    8): T = 300 282 / 256, T = 400 297 / 257, Zipf 288 / 190, T = 500 351 / 260 (a
+//    hot expert's weights are streamed once per 32-row task); at 16 and below the
+//    LDS-streaming gate/up reads weights faster (T = 193: 137 / 160 us), but the
+//    down projection is level from 12 rows on (77 / 77) and far better under
+//    skewed routing (Zipf 56 / 46).  16 experts (96 gate/up tiles): 51 / 58 at 16
+//    rows, 58 / 59 at 19, 65 / 61 at 28.
+//  * run-time-K shapes of 64-row tasks: E = 32, H = I = 2880, T = 512 768 / 312;
+//    E = 128, H = 2048, I = 96, T = 1024 113 / 76; not for matrices so small that
+//    the stage ring's start costs more than the products (H = 96, I = 32: 17 /
+//    20).  Large matrices with fewer rows too: H = I = 2880, E = 32, K = 4: T = 17
+//    gate/up 176 / 170, down 86 / 99 us; T = 64 230 / 185 and 110 / 108; T = 127
+//    477 / 305 per layer; but H = 2048, I = 96: T = 33 44 / 53, T = 100 51 / 60, and
+//    with weight rows a multiple of 4 KiB apart (the tiles' 128-byte pieces then
+//    stream slower) H = 4096, I = 1536, T = 40: gate/up 162 / 180.
+static bool tiled(const ExpertArgs &a, int token_block, int path, bool down, int tiles, int min_rows, int num_cus) {
+  if (path == kTile) return true;
+  if (!tile_gemm_ok(a.H, a.I)) return false;
+  const long long hi = (long long)a.H * a.I, units = (long long)a.E * tiles, rows = a.R;
+  if (path == kStream) {
+    if (rows > 16LL * a.E) return units >= num_cus || (4 * units >= num_cus && rows > 20LL * a.E);
+    return down && rows >= 12LL * a.E && units >= num_cus;
+  }
+  if (path != kGeneric) return false;
+  if (token_block == 64) return hi >= 65536;
+  return hi >= (1 << 20) && units >= num_cus && rows >= (long long)min_rows * a.E;
+}
+static bool tiled_gate_up(const ExpertArgs &a, int token_block, int path, int num_cus) {
+  return tiled(a, token_block, path, false, (a.I + 127) / 128, a.H % 2048 ? 2 : 12, num_cus);
+}
+static bool tiled_down(const ExpertArgs &a, int token_block, int path, int num_cus) {
+  return tiled(a, token_block, path, true, (a.H + 255) / 256, 6, num_cus);
+}
 
 // W4 gate/up of 64-row tasks at H = 2048: the register-streaming pair kernel
 // decodes each weight once per 96 rows, the tiled kernel once per 160 and with
@@ -180,12 +210,12 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   // row per expert the split-K streaming kernel overlaps the decode better, and
   // with the folded decode it is faster for 16-row tasks too (T = 193: gate/up
   // 49 vs 61 us).
-  if (w4 && token_block == 64 && !w4_pair_preferred(a, num_cus) && (path == kTile || generic_tiled(a.H, a.I)))
+  if (w4 && token_block == 64 && !w4_pair_preferred(a, num_cus) && tiled_gate_up(a, token_block, path, num_cus))
     return launch_tile_gate_up(a, true, num_cus, s);
   const bool wave_ok = w4 && (token_block != 64 || a.H == 2048) && wave_w4_shape_ok(a.H, a.I, token_block);
   if (wave_ok && path != kGeneric && (token_block == 64 || ((long long)a.R >= 4LL * a.E && !a.w4_fold)))
     return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (path == kTile) return w4 ? hipErrorInvalidValue : launch_tile_gate_up(a, false, num_cus, s);
+  if (!w4 && tiled_gate_up(a, token_block, path, num_cus)) return launch_tile_gate_up(a, false, num_cus, s);
   if (path == kStream) {
     if (!w4 && kDmaStreaming && dma_shape_ok(a.H, a.I, token_block))
       return launch_dma_gate_up(a, token_block, num_cus, s);
@@ -195,8 +225,6 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
   // fit, else the run-time-K MFMA kernel, else (bf16, H or I not a multiple of
   // 32) the scalar one.
   if (wave_ok) return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (path == kGeneric && token_block == 64 && !w4 && generic_tiled(a.H, a.I))
-    return launch_tile_gate_up(a, false, num_cus, s);
   if (path == kGeneric && flex_shape_ok(a.H, a.I, w4))
     return launch_flex_gate_up(a, task_capacity, token_block, w4, s);
   if (w4) return hipErrorInvalidValue;
@@ -207,13 +235,11 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
 
 hipError_t launch_down(const ExpertArgs &a, int task_capacity, int token_block, int path,
                        int num_cus, hipStream_t s) {
-  if (path == kTile) return launch_tile_down(a, num_cus, s);
+  if (tiled_down(a, token_block, path, num_cus)) return launch_tile_down(a, num_cus, s);
   if (path == kStream) {
     if (kDmaStreaming && kDmaDown && dma_shape_ok(a.H, a.I, token_block)) return launch_dma_down(a, token_block, num_cus, s);
     return launch_stream_down(a, task_capacity, token_block, num_cus, s);
   }
-  if (path == kGeneric && token_block == 64 && generic_tiled(a.H, a.I))
-    return launch_tile_down(a, num_cus, s);
   if (path == kGeneric && flex_shape_ok(a.H, a.I, false))
     return launch_flex_down(a, task_capacity, token_block, s);
   const dim3 grid(task_capacity, (token_block * a.H + 255) / 256);

@@ -158,6 +158,32 @@ def test_tiled_row_blocks(hidden, inter, w4, special, gpu_device):
     assert m["passed"], m
 
 
+@pytest.mark.parametrize("tokens,experts,hidden,inter,topk", [
+    (192, 64, 1024, 512, 4),   # 12 rows per expert, 256 down tiles: streaming gate/up, tiled down
+    (272, 64, 512, 512, 4),    # 17 rows: gate/up tiled (256 tiles), streaming down (128 tiles)
+    (324, 64, 512, 512, 4),    # 20.25 rows: both tiled
+    (100, 32, 2880, 1440, 4),  # run-time-K shape, 32-row tasks, both tiled
+    (17, 32, 2880, 1440, 4),   # about two rows: gate/up tiled, down run-time-K
+    (24, 32, 2048, 1440, 4),   # rows a multiple of 4 KiB apart: run-time-K gate/up
+])
+def test_tiled_rules_below_64_rows(tokens, experts, hidden, inter, topk, gpu_device):
+    """Shapes on both sides of the rules that take 16- and 32-row tasks to the
+    LDS-tiled kernels, through the router, against the FP32 oracle."""
+    x, gu, dn, _, _ = O.make_inputs(tokens=tokens, experts=experts, topk=topk, hidden=hidden, intermediate=inter,
+                                    id_dtype=torch.int32, pattern="random", seed=tokens + hidden)
+    logits = torch.randn((tokens, experts), generator=torch.Generator().manual_seed(tokens))
+    logits[:, 0] += 2.0  # a hot expert: several row blocks
+    xd, gud, dnd, ld = _to(gpu_device, x, gu, dn, logits)
+    plan = prepare_routed_moe(xd, ld, gud, dnd, topk)
+    out = plan.forward(xd, ld)
+    torch.cuda.synchronize()
+    plan.check_inputs()
+    ids, w = O.route_topk(logits, topk)
+    assert torch.equal(plan.ids.cpu(), ids)
+    m = O.error(out, O.moe_reference(x, gu, dn, ids, w))
+    assert m["passed"], m
+
+
 def test_w4_pair_passes_at_task_boundaries(gpu_device):
     """W4 gate/up with 64-row tasks (the pair kernel): experts with 1, 33, 64, 65, 96,
     97, 129 and 160 rows cover a single short task, a full task, two tasks run as one
