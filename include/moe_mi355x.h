@@ -124,9 +124,10 @@ typedef struct moe_layout {
                        * (T <= 32); 5 (separate router launch) only for shapes   *
                        * with more tokens than the planner's workgroups hold     *
                        * (T > 16 x CU count); 0 when T == 0                      */
-  int32_t fast_path;  /* 0 run-time-K MFMA kernels (other shapes; scalar where   
-                         H or I is not a multiple of 32), 1 MFMA weight         
-                         streaming, 2 MFMA LDS-tiled (many rows per expert)     */
+  int32_t fast_path;  /* family by shape: 0 run-time-K MFMA kernels (scalar where
+                         H or I is not a multiple of 32), 1 MFMA weight
+                         streaming, 2 MFMA LDS-tiled (many rows per expert); 0
+                         and 1 run the tiled GEMMs too where those are faster */
 } moe_layout;
 
 typedef struct moe_plan moe_plan;

@@ -656,8 +656,12 @@ int gqa_prefill_splits(int T, int Hq, int Hkv, long long history, int num_cus) {
 }
 
 GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus) {
-  const int G = Hq / Hkv;
   if (const int s = gqa_prefill_splits(T, Hq, Hkv, history, num_cus)) return {s, 12, 2, true};
+  return gqa_short_shape(T, Hq, Hkv, num_cus);
+}
+
+GqaShape gqa_short_shape(int T, int Hq, int Hkv, int num_cus) {
+  const int G = Hq / Hkv;
   const int w1 = gqa_workgroups(T, Hkv, G, 1);
   if (w1 <= 0) return {1, 4, 2, false};
   if (w1 <= num_cus) {

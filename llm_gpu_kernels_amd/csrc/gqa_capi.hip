@@ -98,8 +98,15 @@ int gqa_seg_plan_create(gqa_seg_plan **out, const gqa_seg_desc *d) {
   int rc = device_cus(&dev, &cus);
   if (rc) return rc;
   if ((rc = validate(d, cus, &shape))) return rc;
-  const size_t need = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
-  if (need && (d->workspace_bytes < need || !d->workspace || !aligned16(d->workspace)))
+  size_t need = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
+  auto lacks = [&] { return need && (d->workspace_bytes < need || !d->workspace || !aligned16(d->workspace)); };
+  if (shape.prefill && lacks()) {
+    // Less workspace than gqa_seg_workspace_bytes() asks for: the short-chunk
+    // kernel needs none at these lengths, or less.
+    shape = moe::gqa_short_shape(d->T, d->Hq, d->Hkv, cus);
+    need = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
+  }
+  if (lacks())
     return moe::capi_fail(MOE_ESPACE, "workspace has %zu bytes, needs %zu", d->workspace_bytes,
                           need);
   gqa_seg_plan *p = new (std::nothrow) gqa_seg_plan;

@@ -32,6 +32,9 @@ struct GqaShape {
   bool prefill;
 };
 GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus);
+// The shape without the long-chunk kernel, for callers whose workspace does not
+// hold that kernel's split states.
+GqaShape gqa_short_shape(int T, int Hq, int Hkv, int num_cus);
 // Workgroups of the long-chunk kernel before splitting (256 query rows each).
 int gqa_prefill_workgroups(int T, int Hq, int Hkv);
 hipError_t launch_gqa_prefill(const GqaArgs &a, int nsplit, hipStream_t s);

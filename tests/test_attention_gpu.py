@@ -79,7 +79,7 @@ def test_group_sizes(hq, hkv, gpu_device):
 
 @pytest.mark.parametrize("tokens,hq,hkv,history", [
     (2048, 32, 8, (16, 0, 1)),         # mostly causal, one round of workgroups, no split
-    (530, 32, 8, (8192, 2049, 575)),   # key splits and the merge, ragged last query block
+    (500, 32, 8, (8192, 2049, 575)),   # key splits and the merge, ragged last query block
     (1020, 16, 8, (8000, 100, 3)),     # two heads per KV head
     (2000, 8, 8, (9000, 0, 65)),       # one head per KV head
     (700, 64, 8, (6000, 63, 0)),       # eight heads per KV head, an empty segment
@@ -89,13 +89,32 @@ def test_long_chunks(tokens, hq, hkv, history, gpu_device):
     stages): every group size, short last tiles of each segment, query blocks
     that end inside a workgroup, with and without key splits; repeated runs are
     bitwise equal."""
-    q, segs = _values(tokens, tokens, history, gpu_device, hq=hq, hkv=hkv, v_stride=6144 if tokens == 530 else None)
+    q, segs = _values(tokens, tokens, history, gpu_device, hq=hq, hkv=hkv, v_stride=6144 if tokens == 500 else None)
     plan = prepare_segmented_gqa(q, segs)
     first = plan.run().clone()
     again = plan.run().clone()
     torch.cuda.synchronize()
     assert torch.equal(first.view(torch.int16), again.view(torch.int16))
     _check(first, q, segs)
+
+
+def test_long_chunk_without_split_workspace(gpu_device):
+    """A plan whose workspace does not hold the long-chunk kernel's split states
+    is accepted and runs the kernel that needs none."""
+    import ctypes
+    from llm_gpu_kernels_amd import _native as N
+    q, segs = _values(9, 500, (8192, 2049, 575), gpu_device)
+    plan = prepare_segmented_gqa(q, segs)
+    assert plan.splits_workspace_bytes > 0
+    plan._desc.workspace, plan._desc.workspace_bytes = None, 0
+    handle = ctypes.c_void_p()
+    N.check(N.lib().gqa_seg_plan_create(ctypes.byref(handle), ctypes.byref(plan._desc)), "create")
+    plan.output.zero_()
+    stream = torch.cuda.current_stream(gpu_device).cuda_stream
+    N.check(N.lib().gqa_seg_plan_run(handle, ctypes.c_void_p(stream)), "run")
+    torch.cuda.synchronize()
+    N.lib().gqa_seg_plan_destroy(handle)
+    _check(plan.output, q, segs)
 
 
 def test_split_merge_partial_workgroup(gpu_device):
