@@ -561,6 +561,10 @@ constexpr int kMergeRows = 4;
 // combined in fixed split order, four splits per round trip: the loads of a
 // group are issued together (a plain loop over a run-time count would issue
 // one round trip per split) and the running maximum is rescaled between groups.
+// A split without a visible key (m = -inf) has weight 0, and a row without any
+// is 0; everywhere else, and in the products with a weight of 0, NaN passes
+// through as it does in an unsplit launch (a NaN score leaves m alone and shows
+// in l and O only).
 __global__ __launch_bounds__(128 * kMergeRows) void gqa_merge_kernel(GqaArgs a, int nsplit) {
   constexpr int kGroup = 4;
   const int th = blockIdx.x * kMergeRows + threadIdx.x / kD;  // token * Hq + head
@@ -581,7 +585,6 @@ __global__ __launch_bounds__(128 * kMergeRows) void gqa_merge_kernel(GqaArgs a, 
     float Mn = M;
 #pragma unroll
     for (int j = 0; j < kGroup; ++j) Mn = s0 + j < nsplit ? fmaxf(Mn, m[j]) : Mn;
-    if (Mn == -INFINITY) continue;  // nothing visible so far
     const float r = M == -INFINITY ? 0.f : exp2f(M - Mn);
     num *= r;
     den *= r;
@@ -593,7 +596,7 @@ __global__ __launch_bounds__(128 * kMergeRows) void gqa_merge_kernel(GqaArgs a, 
     }
     M = Mn;
   }
-  const float v = den > 0.f ? num / den : 0.f;
+  const float v = den == 0.f ? num * 0.f : num / den;
   a.out[(int64_t)th * kD + d] = (uint16_t)(pack_bf16x2(v, 0.f) & 0xffffu);
 }
 

@@ -117,6 +117,30 @@ def test_long_chunk_without_split_workspace(gpu_device):
     _check(plan.output, q, segs)
 
 
+@pytest.mark.parametrize("tokens,history", [
+    (32, (1024, 512, 256)),    # short chunk, keys split, merge launch
+    (256, (1024, 512, 256)),   # short chunk, no split
+    (500, (8192, 2049, 575)),  # long chunk, keys split, merge launch
+    (2048, (16, 0, 1)),        # long chunk, no split
+])
+def test_non_finite_scores(tokens, history, gpu_device):
+    """NaN in q or K and scores of +inf give NaN rows exactly where the FP32
+    oracle has them, split or not; scores of -inf drop their key."""
+    q, segs = _values(tokens + 5, tokens, history, gpu_device)
+    q[tokens // 2, 3, 7] = float("nan")          # one row
+    segs[0][0][9, 2, 100] = float("nan")         # every row of KV head 2
+    segs[2][0][0, 7, 31] = float("inf")          # +inf or -inf by the sign of q's element
+    ref = O.gqa_segmented_reference(q.cpu(), [(k.cpu(), v.cpu()) for k, v in segs]).float()
+    segs[-1][0][tokens - 3, 5, 64] = float("nan")  # the last three tokens of KV head 5
+    ref[tokens - 3:, 20:24] = float("nan")         # (the oracle adds its mask: NaN for the tokens before too)
+    out = prepare_segmented_gqa(q, segs).output.cpu().float()
+    nan = ref.isnan()
+    assert 0 < int(nan.sum()) < nan.numel()
+    assert torch.equal(out.isnan(), nan)
+    m = O.error(out.masked_fill(nan, 0.0), ref.masked_fill(nan, 0.0), LIMITS)
+    assert m["passed"], m
+
+
 def test_split_merge_partial_workgroup(gpu_device):
     """T * Hq = 66 (query) rows with the keys split: the merge launch's last
     workgroup holds fewer rows than the others."""
