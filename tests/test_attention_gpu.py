@@ -141,6 +141,33 @@ def test_non_finite_scores(tokens, history, gpu_device):
     assert m["passed"], m
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,history", [
+    (256, 32, 8, (1024, 512, 256)),    # short chunk
+    (500, 32, 8, (8192, 2049, 575)),   # long chunk, keys split
+    (2047, 32, 8, (16, 0, 1)),         # long chunk, no split, 64 tokens per workgroup
+    (2000, 8, 8, (9000, 0, 65)),       # 256 tokens per workgroup
+    (1020, 16, 8, (8000, 100, 3)),     # 128
+    (700, 64, 8, (6000, 63, 0)),       # 32
+])
+def test_non_finite_values_of_later_tokens(tokens, hq, hkv, history, gpu_device):
+    """A row of V that is not finite reaches its own token and the later ones;
+    tokens of earlier 16-token blocks keep their values, those of earlier
+    32-token blocks their bits.  (The long-chunk kernel adds up the 32 tokens
+    around such a row in another order.)"""
+    q, segs = _values(tokens + 6, tokens, history, gpu_device, hq=hq, hkv=hkv)
+    plan = prepare_segmented_gqa(q, segs)
+    clean = plan.output.clone()
+    for row in (tokens - 3, tokens // 2 + 21, tokens // 2 + 5, 40, 17, 0):
+        segs[-1][1][row] = float("inf") if row % 2 else float("nan")
+        out = plan.run()
+        same = row // 32 * 32
+        assert torch.equal(out[:same].view(torch.int16), clean[:same].view(torch.int16)), row
+        if row // 16 * 16 > same:
+            m = O.error(out[same:row // 16 * 16].cpu(), clean[same:row // 16 * 16].cpu().float(), LIMITS)
+            assert m["passed"], (row, m)
+        assert not out[row:].isfinite().any(), row
+
+
 def test_split_merge_partial_workgroup(gpu_device):
     """T * Hq = 66 (query) rows with the keys split: the merge launch's last
     workgroup holds fewer rows than the others."""
