@@ -158,6 +158,31 @@ def test_tiled_row_blocks(hidden, inter, w4, special, gpu_device):
     assert m["passed"], m
 
 
+def test_tiled_swiglu_matches_streaming(gpu_device):
+    """One-hot token rows make gate and up exact, so the activations of the tiled
+    kernels are bit for bit those of the streaming kernels, over every sign and
+    magnitude of the gate (exponentials from subnormal to infinite)."""
+    n = 256
+    gen = torch.Generator().manual_seed(7)
+    gate = (torch.rand((n, n), generator=gen) * 2 - 1) * torch.tensor([1.0, 4.0, 20.0, 110.0]).repeat(n // 4)[:, None]
+    gate[3, :16] = torch.linspace(-89.0, -86.0, 16)
+    gu = torch.cat([gate, torch.randn((n, n), generator=gen)]).to(torch.bfloat16)[None]
+    dn = torch.zeros((1, n, n), dtype=torch.bfloat16)
+    x = torch.eye(n, dtype=torch.bfloat16)
+    ids, w = torch.zeros((n, 1), dtype=torch.int32), torch.ones((n, 1))
+    dev = _to(gpu_device, x, gu, dn, ids, w)
+    tiled = prepare_moe(*dev, config=GemmConfig(block_m=64))
+    streaming = prepare_moe(*dev, config=GemmConfig(block_m=16))
+    torch.cuda.synchronize()
+    g = gu[0, :n].float()
+    act = tiled.activated.cpu()
+    assert torch.equal(act.view(torch.int16), streaming.activated.cpu().view(torch.int16))
+    exact = (g.double() / (1 + torch.exp(-g.double())) * gu[0, n:].double()).t()
+    # One bf16 rounding (2^-9) and a few fp32 ones; below g = -88.7 the exponential
+    # is infinite and 0 stands for at most 110 / 3.4e38 |u|, |u| < 5.
+    assert ((act.double() - exact).abs() <= exact.abs() * 2.0 ** -8 + 2e-36).all()
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,inter,topk", [
     (192, 64, 1024, 512, 4),   # 12 rows per expert, 256 down tiles: streaming gate/up, tiled down
     (272, 64, 512, 512, 4),    # 17 rows: gate/up tiled (256 tiles), streaming down (128 tiles)
