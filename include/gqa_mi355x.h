@@ -45,7 +45,14 @@ typedef struct gqa_seg_desc {
 
 typedef struct gqa_seg_plan gqa_seg_plan;
 
-/* Workspace bytes the plan needs on the current device (0 when unsplit). */
+/*
+ * Workspace bytes for the plan on the current device: 520 bytes per token,
+ * head and key split (0 without splits; tens of MB for chunks of hundreds of
+ * tokens against long histories).  A workspace of this size is enough for
+ * every history of the same T, Hq and Hkv: a plan that would split into more
+ * runs the kernel that does with less.  It is scratch of a run: plans that
+ * share one must run in stream order.
+ */
 int gqa_seg_workspace_bytes(const gqa_seg_desc *d, size_t *bytes);
 int gqa_seg_plan_create(gqa_seg_plan **out, const gqa_seg_desc *d);
 /* Enqueue on `stream` (hipStream_t); no sync, no allocation; T == 0 launches nothing. */

@@ -86,7 +86,11 @@ int gqa_seg_workspace_bytes(const gqa_seg_desc *d, size_t *bytes) {
   if (rc) return rc;
   if ((rc = validate(d, cus, &shape))) return rc;
   if (!bytes) return moe::capi_fail(MOE_EINVAL, "null bytes");
-  *bytes = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
+  // At least what the short-chunk kernel needs, which does not depend on the
+  // history: a workspace sized with any history then serves every other.
+  const size_t own = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
+  const size_t any = moe::gqa_partial_bytes(d->T, d->Hq, moe::gqa_short_shape(d->T, d->Hq, d->Hkv, cus).nsplit);
+  *bytes = own > any ? own : any;
   return MOE_OK;
 }
 

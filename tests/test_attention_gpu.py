@@ -98,6 +98,33 @@ def test_long_chunks(tokens, hq, hkv, history, gpu_device):
     _check(first, q, segs)
 
 
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (8, 1), (4, 4), (1, 1)])
+def test_workspace_serves_every_history(hq, hkv, gpu_device):
+    """A workspace sized with one history is accepted with every other history of
+    the same chunk length and heads, whichever kernels the two choose."""
+    import ctypes
+    from llm_gpu_kernels_amd import _native as N
+    base = 1 << 20  # addresses that are only looked at by the validation
+    for tokens in (32, 256, 512, 1024, 2048):
+        descs, sizes = [], []
+        for history in (0, 300, 2000, 9000, 40000):
+            d = N.GqaDesc()
+            d.T, d.Hq, d.Hkv, d.D, d.num_segments = tokens, hq, hkv, 128, 2
+            for i, length in enumerate((history, tokens)):
+                d.len[i], d.k[i], d.v[i] = length, base, base
+                d.k_stride[i] = d.v_stride[i] = hkv * 128
+            d.q = d.out = d.workspace = base
+            size = ctypes.c_size_t()
+            N.check(N.lib().gqa_seg_workspace_bytes(ctypes.byref(d), ctypes.byref(size)), "size")
+            descs.append(d)
+            sizes.append(size.value)
+        for d in descs:
+            for d.workspace_bytes in sizes:
+                handle = ctypes.c_void_p()
+                N.check(N.lib().gqa_seg_plan_create(ctypes.byref(handle), ctypes.byref(d)), "create")
+                N.lib().gqa_seg_plan_destroy(handle)
+
+
 def test_long_chunk_without_split_workspace(gpu_device):
     """A plan whose workspace does not hold the long-chunk kernel's split states
     is accepted and runs the kernel that needs none."""
