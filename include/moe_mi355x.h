@@ -137,6 +137,13 @@ const char *moe_last_error(void);
 
 /* Workspace size and layout for a descriptor (pointers may be NULL). */
 int moe_workspace_layout(const moe_desc *d, moe_layout *out);
+/* Kernels that a forward of this shape takes on a GPU of num_cus compute units,
+ * aligned buffers assumed (pointers may be NULL; host only, for tests and
+ * measurements): out = {gate/up kernel, its token rows per unit at most, down
+ * kernel, its rows}.  No counterpart in the reference. */
+enum { MOE_GEMM_SCALAR = 0, MOE_GEMM_RUNTIME_K = 1, MOE_GEMM_STREAM = 2, MOE_GEMM_LDS_STREAM = 3,
+       MOE_GEMM_DECODE_ONCE = 4, MOE_GEMM_TILED = 5 };
+int moe_gemm_choice(const moe_desc *d, int32_t num_cus, int32_t out[4]);
 
 /* Validate the descriptor and bind its pointers.  No allocation, no launch,
  * no device work (so it may run during stream capture).  The workspace must

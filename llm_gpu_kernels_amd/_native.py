@@ -19,6 +19,7 @@ MOE_OK, MOE_EINVAL, MOE_EDEVICE, MOE_ESPACE = 0, -1, -2, -3
 WEIGHTS_BF16, WEIGHTS_W4G128, WEIGHTS_W4G128_FOLD = 0, 1, 2
 IDS_INT32, IDS_INT64 = 0, 1
 ROUTE_FIXED, ROUTE_LOGITS = 0, 1
+GEMM_SCALAR, GEMM_RUNTIME_K, GEMM_STREAM, GEMM_LDS_STREAM, GEMM_DECODE_ONCE, GEMM_TILED = range(6)
 STATUS_BAD_ID, STATUS_BAD_WEIGHT, STATUS_BAD_LOGIT, STATUS_DIRTY_COUNTERS, STATUS_STALLED = 1, 2, 4, 8, 16
 
 
@@ -60,6 +61,7 @@ SIGNATURES = {
     "moe_abi_version": (c_int32, []),
     "moe_last_error": (ctypes.c_char_p, []),
     "moe_workspace_layout": (c_int32, [POINTER(MoeDesc), POINTER(MoeLayout)]),
+    "moe_gemm_choice": (c_int32, [POINTER(MoeDesc), c_int32, POINTER(c_int32)]),
     "moe_plan_create": (c_int32, [POINTER(c_void_p), POINTER(MoeDesc)]),
     "moe_plan_run": (c_int32, [c_void_p, c_void_p]),
     "moe_plan_run_stage": (c_int32, [c_void_p, c_int32, c_void_p]),

@@ -184,6 +184,11 @@ int capi_fail(int code, const char *fmt, ...) {
 }
 }  // namespace moe
 
+static_assert(moe::kScalarGemm == MOE_GEMM_SCALAR && moe::kFlexGemm == MOE_GEMM_RUNTIME_K &&
+                  moe::kStreamGemm == MOE_GEMM_STREAM && moe::kDmaGemm == MOE_GEMM_LDS_STREAM &&
+                  moe::kWaveGemm == MOE_GEMM_DECODE_ONCE && moe::kTileGemm == MOE_GEMM_TILED,
+              "kernel numbers of the header");
+
 struct moe_plan {
   moe_desc d;
   moe_layout L;
@@ -287,6 +292,21 @@ int moe_workspace_layout(const moe_desc *d, moe_layout *out) {
   if (rc) return rc;
   if (!out) return fail(MOE_EINVAL, "null layout");
   *out = compute_layout(d);
+  return MOE_OK;
+}
+
+int moe_gemm_choice(const moe_desc *d, int32_t num_cus, int32_t out[4]) {
+  int rc = validate(d);
+  if (rc) return rc;
+  if (!out || num_cus < 1) return fail(MOE_EINVAL, "null output or no compute units");
+  const int tb = choose_token_block(d), path = choose_path(d, tb);
+  moe::ExpertArgs a{};
+  a.T = d->T, a.H = d->H, a.I = d->I, a.E = d->E, a.K = d->K, a.R = d->T * d->K;
+  a.w4_fold = d->weight_format == MOE_WEIGHTS_W4G128_FOLD;
+  out[0] = moe::gate_up_kernel(a, tb, is_w4(d->weight_format), path, num_cus);
+  out[1] = out[0] == moe::kTileGemm ? moe::tile_unit_rows(a, false, num_cus) : tb;
+  out[2] = moe::down_kernel(a, tb, path, num_cus);
+  out[3] = out[2] == moe::kTileGemm ? moe::tile_unit_rows(a, true, num_cus) : tb;
   return MOE_OK;
 }
 

@@ -203,31 +203,46 @@ static bool w4_pair_preferred(const ExpertArgs &a, int num_cus) {
   return a.H == 2048 && (long long)a.R < 128LL * a.E && (long long)a.E * ((a.I + 255) / 256) * 4 >= num_cus;
 }
 
-hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_block, bool w4,
-                          int path, int num_cus, hipStream_t s) {
+GemmKernel gate_up_kernel(const ExpertArgs &a, int token_block, bool w4, int path, int num_cus) {
   // W4 with several rows per expert, and every 64-row task: decode each weight
   // fragment once for up to 64 token rows (one unit per wave).  With about one
   // row per expert the split-K streaming kernel overlaps the decode better, and
   // with the folded decode it is faster for 16-row tasks too (T = 193: gate/up
   // 49 vs 61 us).
   if (w4 && token_block == 64 && !w4_pair_preferred(a, num_cus) && tiled_gate_up(a, token_block, path, num_cus))
-    return launch_tile_gate_up(a, true, num_cus, s);
+    return kTileGemm;
   const bool wave_ok = w4 && (token_block != 64 || a.H == 2048) && wave_w4_shape_ok(a.H, a.I, token_block);
   if (wave_ok && path != kGeneric && (token_block == 64 || ((long long)a.R >= 4LL * a.E && !a.w4_fold)))
-    return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (!w4 && tiled_gate_up(a, token_block, path, num_cus)) return launch_tile_gate_up(a, false, num_cus, s);
-  if (path == kStream) {
-    if (!w4 && kDmaStreaming && dma_shape_ok(a.H, a.I, token_block))
-      return launch_dma_gate_up(a, token_block, num_cus, s);
-    return launch_stream_gate_up(a, task_capacity, token_block, w4, num_cus, s);
-  }
+    return kWaveGemm;
+  if (!w4 && tiled_gate_up(a, token_block, path, num_cus)) return kTileGemm;
+  if (path == kStream)
+    return !w4 && kDmaStreaming && dma_shape_ok(a.H, a.I, token_block) ? kDmaGemm : kStreamGemm;
   // Shapes the tuned kernels do not take: the W4 wave kernel where its K-chunks
   // fit, else the run-time-K MFMA kernel, else (bf16, H or I not a multiple of
   // 32) the scalar one.
-  if (wave_ok) return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
-  if (path == kGeneric && flex_shape_ok(a.H, a.I, w4))
-    return launch_flex_gate_up(a, task_capacity, token_block, w4, s);
-  if (w4) return hipErrorInvalidValue;
+  if (wave_ok) return kWaveGemm;
+  if (path == kGeneric && flex_shape_ok(a.H, a.I, w4)) return kFlexGemm;
+  return w4 ? kNoGemm : kScalarGemm;
+}
+
+GemmKernel down_kernel(const ExpertArgs &a, int token_block, int path, int num_cus) {
+  if (tiled_down(a, token_block, path, num_cus)) return kTileGemm;
+  if (path == kStream)
+    return kDmaStreaming && kDmaDown && dma_shape_ok(a.H, a.I, token_block) ? kDmaGemm : kStreamGemm;
+  return path == kGeneric && flex_shape_ok(a.H, a.I, false) ? kFlexGemm : kScalarGemm;
+}
+
+hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_block, bool w4,
+                          int path, int num_cus, hipStream_t s) {
+  switch (gate_up_kernel(a, token_block, w4, path, num_cus)) {
+    case kTileGemm: return launch_tile_gate_up(a, w4, num_cus, s);
+    case kWaveGemm: return launch_wave_w4_gate_up(a, task_capacity, token_block, s);
+    case kDmaGemm: return launch_dma_gate_up(a, token_block, num_cus, s);
+    case kStreamGemm: return launch_stream_gate_up(a, task_capacity, token_block, w4, num_cus, s);
+    case kFlexGemm: return launch_flex_gate_up(a, task_capacity, token_block, w4, s);
+    case kScalarGemm: break;
+    default: return hipErrorInvalidValue;
+  }
   const dim3 grid(task_capacity, (token_block * a.I + 255) / 256);
   hipLaunchKernelGGL(gate_up_generic_kernel, grid, dim3(256), 0, s, a, token_block);
   return hipGetLastError();
@@ -235,13 +250,13 @@ hipError_t launch_gate_up(const ExpertArgs &a, int task_capacity, int token_bloc
 
 hipError_t launch_down(const ExpertArgs &a, int task_capacity, int token_block, int path,
                        int num_cus, hipStream_t s) {
-  if (tiled_down(a, token_block, path, num_cus)) return launch_tile_down(a, num_cus, s);
-  if (path == kStream) {
-    if (kDmaStreaming && kDmaDown && dma_shape_ok(a.H, a.I, token_block)) return launch_dma_down(a, token_block, num_cus, s);
-    return launch_stream_down(a, task_capacity, token_block, num_cus, s);
+  switch (down_kernel(a, token_block, path, num_cus)) {
+    case kTileGemm: return launch_tile_down(a, num_cus, s);
+    case kDmaGemm: return launch_dma_down(a, token_block, num_cus, s);
+    case kStreamGemm: return launch_stream_down(a, task_capacity, token_block, num_cus, s);
+    case kFlexGemm: return launch_flex_down(a, task_capacity, token_block, s);
+    default: break;
   }
-  if (path == kGeneric && flex_shape_ok(a.H, a.I, false))
-    return launch_flex_down(a, task_capacity, token_block, s);
   const dim3 grid(task_capacity, (token_block * a.H + 255) / 256);
   hipLaunchKernelGGL(down_generic_kernel, grid, dim3(256), 0, s, a, token_block);
   return hipGetLastError();

@@ -96,6 +96,8 @@ hipError_t launch_wave_w4_gate_up(const ExpertArgs &a, int task_capacity, int to
 hipError_t launch_tile_gate_up(const ExpertArgs &a, bool w4, int num_cus, hipStream_t s);
 hipError_t launch_tile_down(const ExpertArgs &a, int num_cus, hipStream_t s);
 bool tile_gemm_ok(int H, int I);
+// Token rows of a unit at most.
+int tile_unit_rows(const ExpertArgs &a, bool down, int num_cus);
 // Shapes that report the tiled family (moe_layout.fast_path 2).
 bool tile_shape_ok(int H, int I, bool w4);
 
@@ -104,6 +106,10 @@ bool tile_shape_ok(int H, int I, bool w4);
 // kernels where tile_gemm_ok (or scalar kernels where H or I is not a multiple
 // of 32); kScalar: the scalar kernels (unaligned bf16 buffers).
 enum Path { kGeneric = 0, kStream = 1, kTile = 2, kScalar = 3 };
+// The kernel that launch_gate_up and launch_down take (MOE_GEMM_* of the C ABI).
+enum GemmKernel { kNoGemm = -1, kScalarGemm, kFlexGemm, kStreamGemm, kDmaGemm, kWaveGemm, kTileGemm };
+GemmKernel gate_up_kernel(const ExpertArgs &a, int token_block, bool w4, int path, int num_cus);
+GemmKernel down_kernel(const ExpertArgs &a, int token_block, int path, int num_cus);
 // MFMA kernels for any H, I that are multiples of 32 (W4: H of 128) -- the
 // shapes the tuned kernels above do not take (kGeneric path).
 bool flex_shape_ok(int H, int I, bool w4);

@@ -688,24 +688,38 @@ hipError_t launch_nbm(const ExpertArgs &a, int max_rows, int num_cus, hipStream_
 // 334 us per layer at E = 128, H = 2048, I = 768, K = 8, T = 2048 (mean 128)
 // and 425 vs 448 at E = 32, H = I = 2880, K = 4, T = 1024 (Zipf routing).
 // Below a mean of 128 rows 96-row units waste less of the last round: T = 1024
-// Zipf 242 vs 255 us, uniform 266 vs 267 (64-row units: 262 and 293).  While
-// the units leave half the CUs idle, lower ones: the four-slot ring of 64 rows
-// (16 experts of 64 rows: 66.3 vs 67.9 us), then 32-row units where an
-// expert's rows still make more of them (E = 8, H = 512, I = 256, 256 rows
-// each: 26.5 vs 28.3 us).
+// Zipf 242 vs 255 us, uniform 266 vs 267 (64-row units: 262 and 293).  Where the
+// units of the mean expert leave half the CUs idle, lower ones that make more
+// of them: the four-slot ring of 64 rows (16 experts, H = 2048, I = 768, 64
+// rows each: 66.3 vs 67.9 us; 88 rows 71.3 -> 67.6 for the down projection), 96
+// instead of 160 rows where one block holds the whole expert (128 rows each:
+// 82.2 -> 73.1 us), then 32-row units where an expert's rows still make more of
+// them (E = 8, H = 512, I = 256, 256 rows each: 26.5 vs 28.3 us).  Two 64-row
+// blocks also where they leave a quarter of one round for the experts above
+// the mean (16 experts of 100 / 127 rows, gate/up: 75.5 -> 70.5 / 73.5 -> 71.9 us;
+// with less to spare they start a second round: down at 127 rows 73.5 -> 80.9).
 int unit_blocks(long long R, int E, int ntiles, int num_cus) {
   const long long mean = (R + E - 1) / E;
   auto units = [&](int nb) { return (long long)E * ntiles * ((mean + 32 * nb - 1) / (32 * nb)); };
   int nb = mean >= 128 ? kMaxNB : mean > 40 ? 3 : 2;
   if (nb == 3 && mean <= 64 && 2 * units(2) <= num_cus) nb = 2;
-  while (nb > 1 && mean > (nb > 2 ? 32 : 64) * (nb - 1) && 2 * units(nb) < num_cus) --nb;
+  if (nb == 3 && mean > 96 && 4 * units(2) <= 3LL * num_cus) nb = 2;
+  while (2 * units(nb) <= num_cus) {
+    int n = nb - 1;
+    while (n > 1 && units(n) == units(nb)) --n;  // the next height that makes more units
+    if (n < 1 || (n == 1 && (mean <= 64 || 2 * units(nb) == num_cus))) break;
+    nb = n;
+  }
   return nb;
+}
+
+int unit_blocks(const ExpertArgs &a, bool down, int num_cus) {
+  return unit_blocks(a.R, a.E, down ? (a.H + kBN - 1) / kBN : (a.I + kBN / 2 - 1) / (kBN / 2), num_cus);
 }
 
 template <int KIND, bool W4>
 hipError_t launch_tile(const ExpertArgs &a, int num_cus, hipStream_t s) {
-  const int ntiles = KIND == 0 ? (a.I + kBN / 2 - 1) / (kBN / 2) : (a.H + kBN - 1) / kBN;
-  const int nb = unit_blocks(a.R, a.E, ntiles, num_cus);
+  const int nb = unit_blocks(a, KIND == 1, num_cus);
   if (nb <= 2) return launch_nbm<KIND, 2, W4>(a, 32 * nb, num_cus, s);
   // W4 loads (and zero-fills) NBM token blocks per stage.
   if (W4 && nb == 3) return launch_nbm<KIND, W4 ? 3 : kMaxNB, W4>(a, 32 * nb, num_cus, s);
@@ -724,6 +738,8 @@ bool tile_shape_ok(int H, int I, bool w4) {
   if (I % 128 || H % 256 || !tile_gemm_ok(H, I)) return false;
   return w4 ? wave_w4_shape_ok(H, I, 64) : true;  // W4 gate/up runs in the wave kernel
 }
+
+int tile_unit_rows(const ExpertArgs &a, bool down, int num_cus) { return 32 * unit_blocks(a, down, num_cus); }
 
 hipError_t launch_tile_gate_up(const ExpertArgs &a, bool w4, int num_cus, hipStream_t s) {
   return w4 ? launch_tile<0, true>(a, num_cus, s) : launch_tile<0, false>(a, num_cus, s);

@@ -102,6 +102,33 @@ def test_layout_for_qwen_shape():
     assert rc == 0 and lay.fast_path == 0
 
 
+def _choice(cus=256, **kw):
+    out = (ctypes.c_int32 * 4)()
+    assert N.lib().moe_gemm_choice(ctypes.byref(_desc(**kw)), cus, out) == 0, N.last_error()
+    return list(out)
+
+
+@pytest.mark.parametrize("fmt", [N.WEIGHTS_BF16, N.WEIGHTS_W4G128])
+@pytest.mark.parametrize("experts", [1, 8, 16, 32, 128])
+def test_tiled_units_fill_idle_cus(experts, fmt):
+    """While the units of the mean expert leave half the CUs idle, lower ones
+    that make more of them are taken: never fewer units with more rows, also
+    where one block holds the whole expert (a mean of 128 rows)."""
+    def units(inter, mean, rows):
+        return experts * (-(-inter // 128)) * (-(-mean // rows))
+    for inter in (96, 256, 512, 768, 1536):
+        for mean in list(range(100, 170)) + [192, 256, 320, 321]:
+            kernel, rows, _, _ = _choice(T=mean * experts, K=1, E=experts, H=1024, I=inter, fmt=fmt, tb=64)
+            assert kernel == N.GEMM_TILED and rows in (32, 64, 96, 128, 160)
+            n = units(inter, mean, rows)
+            assert 2 * n >= 256 or n == units(inter, mean, 32), (inter, mean, rows)
+    # 16 experts, gate/up and down (six and eight weight tiles).
+    rows = {t: _choice(T=t, K=1, E=16, fmt=fmt)[1::2] for t in (1024, 1400, 1600, 2032, 2048, 2049, 4096)}
+    assert rows == {1024: [64, 64], 1400: [64, 64], 1600: [64, 96], 2032: [64, 96], 2048: [96, 96],
+                    2049: [128, 128], 4096: [160, 160]}
+    assert _choice(T=2048, fmt=fmt)[1] == 160  # every CU has units: the fewest weight reads
+
+
 @pytest.mark.parametrize("kw", [dict(E=0), dict(E=257), dict(K=0), dict(K=33), dict(H=0),
                                 dict(I=-1), dict(T=-1), dict(fmt=7), dict(ids=9), dict(tb=8), dict(tb=48),
                                 dict(route=N.ROUTE_LOGITS, ids=N.IDS_INT64),
