@@ -54,6 +54,10 @@ typedef struct gqa_seg_plan gqa_seg_plan;
  * share one must run in stream order.
  */
 int gqa_seg_workspace_bytes(const gqa_seg_desc *d, size_t *bytes);
+/* What a plan runs on a GPU of num_cus compute units, with a workspace of that
+ * size (host only, for tests and measurements; buffers as for a plan): out =
+ * {1 long-chunk kernel, 0 short-chunk kernel; key splits}. */
+int gqa_seg_choice(const gqa_seg_desc *d, int32_t num_cus, int32_t out[2]);
 int gqa_seg_plan_create(gqa_seg_plan **out, const gqa_seg_desc *d);
 /* Enqueue on `stream` (hipStream_t); no sync, no allocation; T == 0 launches nothing. */
 int gqa_seg_plan_run(gqa_seg_plan *p, void *stream);

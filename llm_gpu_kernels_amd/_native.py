@@ -77,6 +77,7 @@ SIGNATURES = {
     "moe_w4_dequantize": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p,
                                     c_void_p]),
     "gqa_seg_workspace_bytes": (c_int32, [POINTER(GqaDesc), POINTER(c_size_t)]),
+    "gqa_seg_choice": (c_int32, [POINTER(GqaDesc), c_int32, POINTER(c_int32)]),
     "gqa_seg_plan_create": (c_int32, [POINTER(c_void_p), POINTER(GqaDesc)]),
     "gqa_seg_plan_run": (c_int32, [c_void_p, c_void_p]),
     "gqa_seg_plan_destroy": (None, [c_void_p]),

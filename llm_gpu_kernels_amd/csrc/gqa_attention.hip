@@ -611,31 +611,32 @@ int gqa_workgroups(int T, int Hkv, int G, int rb) {
   return ((T + qt - 1) / qt) * Hkv * (G / hpw);
 }
 
-// Launch shape.  While workgroups of one 16-row block per wave (RB = 1) fit
-// the CUs once, those: the per-step chain of each wave is half as long and
-// twice as many CUs work.  Eight-wave workgroups when they fill more than half
-// the CUs, else four-wave ones with the keys split across up to four
-// workgroups (256 CUs, config-5 heads: T = 16 / 32 / 48 / 64 / 96 / 128 take
-// 10.4 / 11.4 / 14.0 / 14.6 / 15.4 / 15.7 us against 13.7 / 14.1 / 16.0 /
-// 16.3 / 16.8 / 17.1 us with RB = 2).  Beyond that two row blocks per wave
-// (RB = 2, each K/V step shared by 32 rows): with enough workgroups for two
-// per CU, four-wave workgroups and no split; otherwise eight-wave
-// workgroups, one per CU, and the keys split half as many times as would fill
-// the CUs (the merge launch and its partial states cost more than idle CUs).
 // Key splits of the long-chunk kernel where it is expected to be faster than the
-// shapes below, else 0.  Times in ns, fitted on 256 CUs for T >= 256.  That
+// shapes below, else 0.  Times in ns, fitted on 256 CUs at 32 / 8 heads and T >=
+// 256 (both kernels measured at 32 / 8, 16 / 8, 8 / 8, 64 / 8, 8 / 1 and 4 / 4).  That
 // kernel takes 6 us + 1.43 us per 64-key stage, up to 1.85 with every CU busy
-// (clocks); its workgroups
-// start with the last query blocks, so with R rounds of them the busiest CU
-// runs the first block or R middle ones; a split adds the merge launch and
-// its partial states.  The kernel of this file takes 10 us + 10 ns per token +
-// 1 us per 790 MFLOP.  Measured (T x history, 32 / 8 heads; this file -> long
-// chunk): 2048 x 10816 510 -> 378 us, 2048 x 1792 148 -> 114, 2048 x 17 81 -> 65,
-// 1500 x 4100 168 -> 148, 1024 x 10816 249 -> 202 (two splits), 512 x 10816 134
-// -> 113 (four); 1024 x 1792 68 -> 68, 512 x 1792 32 -> 41, 256 x 4096 35 -> 44.
-int gqa_prefill_splits(int T, int Hq, int Hkv, long long history, int num_cus) {
-  const int wp = gqa_prefill_workgroups(T, Hq, Hkv);
+// (clocks); its workgroups start with the last query blocks, so with R rounds of
+// them the busiest CU runs the first block or R middle ones; a split adds the
+// merge launch and its partial states, and 5 us per further round that it
+// makes, whose blocks are of very different lengths (T = 3000 against 17 keys, 16 /
+// 8 heads: three splits 87 us, the kernel of this file 71; 4096 against 500, 4 / 4:
+// six splits 54, four 47).  With fewer than seven stages its start does not
+// pay (256 x 17: 12 us against 18).  The kernel of this file takes 10 us + 10 ns
+// per token + 1 us per 790 MFLOP.  Measured (T x history, 32 / 8 heads; this file
+// -> long chunk): 2048 x 10816 508 -> 376 us, 2048 x 1792 143 -> 110, 2048 x 17 82 ->
+// 62, 1500 x 4096 166 -> 142, 1024 x 10816 257 -> 198 (two splits), 512 x 10816 131
+// -> 105 (four); 1024 x 1792 64 -> 73, 512 x 1792 31 -> 38, 256 x 4096 33 -> 38.  With
+// few heads the per-token term is high and the rule up to 12 % off: 4096 x 500, 8 /
+// 1 heads 84 -> 94, 8 / 8 77 -> 81.
+int gqa_prefill_splits(const int *len, int nseg, int Hq, int Hkv, int num_cus) {
+  const int T = len[nseg - 1], wp = gqa_prefill_workgroups(T, Hq, Hkv);
   if (wp <= 0 || T < 256) return 0;
+  long long history = 0, stages = (T + 63) / 64;
+  for (int i = 0; i + 1 < nseg; ++i) {
+    history += len[i];
+    stages += ((long long)len[i] + 63) / 64;
+  }
+  if (stages < 7) return 0;
   const int nqb = wp / Hkv, qt = 256 / (Hq / Hkv);
   const double flops = 512.0 * Hq * ((double)T * history + 0.5 * T * (T + 1.0));
   double best = 0.97 * (10e3 + 10.0 * T + flops / 790e3);
@@ -649,7 +650,7 @@ int gqa_prefill_splits(int T, int Hq, int Hkv, long long history, int num_cus) {
     const double middle = rounds > 1 ? rounds * (double)(history + T - mid * qt) / 64.0 / s : 0.0;
     const double busy = rounds > 1 ? 1.0 : (double)wgs / num_cus;
     double t = 6e3 + (longest > middle ? longest : middle) * (1430.0 + 420.0 * busy);
-    if (s > 1) t += 10e3 + (double)T * Hq * s * 1040.0 / 4e3;
+    if (s > 1) t += 10e3 + (double)T * Hq * s * 1040.0 / 4e3 + 5e3 * (rounds - 1);
     if (t < best) {
       best = t;
       pick = s;
@@ -658,11 +659,22 @@ int gqa_prefill_splits(int T, int Hq, int Hkv, long long history, int num_cus) {
   return pick;
 }
 
-GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus) {
-  if (const int s = gqa_prefill_splits(T, Hq, Hkv, history, num_cus)) return {s, 12, 2, true};
-  return gqa_short_shape(T, Hq, Hkv, num_cus);
+GqaShape gqa_shape(const int *len, int nseg, int Hq, int Hkv, int num_cus) {
+  if (const int s = gqa_prefill_splits(len, nseg, Hq, Hkv, num_cus)) return {s, 12, 2, true};
+  return gqa_short_shape(len[nseg - 1], Hq, Hkv, num_cus);
 }
 
+// Launch shape.  While workgroups of one 16-row block per wave (RB = 1) fit
+// the CUs once, those: the per-step chain of each wave is half as long and
+// twice as many CUs work.  Eight-wave workgroups when they fill more than half
+// the CUs, else four-wave ones with the keys split across up to four
+// workgroups (256 CUs, config-5 heads: T = 16 / 32 / 48 / 64 / 96 / 128 take
+// 10.4 / 11.4 / 14.0 / 14.6 / 15.4 / 15.7 us against 13.7 / 14.1 / 16.0 /
+// 16.3 / 16.8 / 17.1 us with RB = 2).  Beyond that two row blocks per wave
+// (RB = 2, each K/V step shared by 32 rows): with enough workgroups for two
+// per CU, four-wave workgroups and no split; otherwise eight-wave
+// workgroups, one per CU, and the keys split half as many times as would fill
+// the CUs (the merge launch and its partial states cost more than idle CUs).
 GqaShape gqa_short_shape(int T, int Hq, int Hkv, int num_cus) {
   const int G = Hq / Hkv;
   const int w1 = gqa_workgroups(T, Hkv, G, 1);

@@ -26,6 +26,7 @@ struct gqa_seg_plan {
 namespace {
 
 constexpr int64_t kMaxTokenStride = 1LL << 25;
+static_assert(63 * 2 * kMaxTokenStride + 256 < 1LL << 32, "a 64-row stage of the long-chunk kernel");
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -53,7 +54,7 @@ int validate(const gqa_seg_desc *d, int num_cus, moe::GqaShape *shape) {
         d->v_stride[s] % 8)
       return capi_fail(MOE_EINVAL, "segment %d token stride must be >= %lld and a multiple of 8",
                        s, (long long)minst);
-    // The kernel addresses 32 consecutive rows with 32-bit byte offsets.
+    // The kernels address up to 64 consecutive rows with 32-bit byte offsets.
     if (d->k_stride[s] > kMaxTokenStride || d->v_stride[s] > kMaxTokenStride)
       return capi_fail(MOE_EINVAL, "segment %d token stride must be <= %lld elements", s,
                        (long long)kMaxTokenStride);
@@ -62,9 +63,7 @@ int validate(const gqa_seg_desc *d, int num_cus, moe::GqaShape *shape) {
     return capi_fail(MOE_EINVAL, "q/out must be non-null and 16-byte aligned");
   if ((long long)d->T * d->Hq * 128 >= (1LL << 31))
     return capi_fail(MOE_EINVAL, "T * Hq * 128 must be < 2^31");
-  long long history = 0;
-  for (int s = 0; s + 1 < d->num_segments; ++s) history += d->len[s];
-  *shape = moe::gqa_shape(d->T, d->Hq, d->Hkv, history, num_cus);
+  *shape = moe::gqa_shape(d->len, d->num_segments, d->Hq, d->Hkv, num_cus);
   return MOE_OK;
 }
 
@@ -91,6 +90,15 @@ int gqa_seg_workspace_bytes(const gqa_seg_desc *d, size_t *bytes) {
   const size_t own = moe::gqa_partial_bytes(d->T, d->Hq, shape.nsplit);
   const size_t any = moe::gqa_partial_bytes(d->T, d->Hq, moe::gqa_short_shape(d->T, d->Hq, d->Hkv, cus).nsplit);
   *bytes = own > any ? own : any;
+  return MOE_OK;
+}
+
+int gqa_seg_choice(const gqa_seg_desc *d, int32_t num_cus, int32_t out[2]) {
+  moe::GqaShape shape{1, 4, 2, false};
+  if (const int rc = validate(d, num_cus, &shape)) return rc;
+  if (!out || num_cus < 1) return moe::capi_fail(MOE_EINVAL, "null output or no compute units");
+  out[0] = shape.prefill;
+  out[1] = shape.nsplit;
   return MOE_OK;
 }
 

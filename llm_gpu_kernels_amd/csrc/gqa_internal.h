@@ -31,7 +31,7 @@ struct GqaShape {
   int rb;
   bool prefill;
 };
-GqaShape gqa_shape(int T, int Hq, int Hkv, long long history, int num_cus);
+GqaShape gqa_shape(const int *len, int nseg, int Hq, int Hkv, int num_cus);  // segment lengths, T last
 // The shape without the long-chunk kernel, for callers whose workspace does not
 // hold that kernel's split states.
 GqaShape gqa_short_shape(int T, int Hq, int Hkv, int num_cus);

@@ -5,10 +5,12 @@ Cases follow tests/e2e/test_compact_attention.py of the reference (history
 token stride 6144; graph replay after in-place updates; non-default stream)
 and BASELINE config 5 (history 1024/512/256, T in {32, 96, 256}).
 """
+import ctypes
+
 import pytest
 import torch
 
-from llm_gpu_kernels_amd import prepare_segmented_gqa, prepare_cuda_gqa_compact
+from llm_gpu_kernels_amd import _native as N, prepare_segmented_gqa, prepare_cuda_gqa_compact
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -29,6 +31,14 @@ def _values(seed, tokens, history, device, v_stride=None, hq=32, hkv=8):
         pv.copy_(v)
         segs[-1] = (k, pv)
     return q, segs
+
+
+def _long_chunk(plan, device):
+    """{1 long-chunk kernel, 0 short-chunk kernel; key splits} of a plan."""
+    out = (ctypes.c_int32 * 2)()
+    N.check(N.lib().gqa_seg_choice(ctypes.byref(plan._desc),
+                                   torch.cuda.get_device_properties(device).multi_processor_count, out), "choice")
+    return tuple(out)
 
 
 def _check(out, q, segs):
@@ -91,6 +101,8 @@ def test_long_chunks(tokens, hq, hkv, history, gpu_device):
     bitwise equal."""
     q, segs = _values(tokens, tokens, history, gpu_device, hq=hq, hkv=hkv, v_stride=6144 if tokens == 500 else None)
     plan = prepare_segmented_gqa(q, segs)
+    chosen, splits = _long_chunk(plan, gpu_device)
+    assert chosen and (splits > 1) == (tokens in (500, 1020, 2000))
     first = plan.run().clone()
     again = plan.run().clone()
     torch.cuda.synchronize()
@@ -102,8 +114,6 @@ def test_long_chunks(tokens, hq, hkv, history, gpu_device):
 def test_workspace_serves_every_history(hq, hkv, gpu_device):
     """A workspace sized with one history is accepted with every other history of
     the same chunk length and heads, whichever kernels the two choose."""
-    import ctypes
-    from llm_gpu_kernels_amd import _native as N
     base = 1 << 20  # addresses that are only looked at by the validation
     for tokens in (32, 256, 512, 1024, 2048):
         descs, sizes = [], []
@@ -128,8 +138,6 @@ def test_workspace_serves_every_history(hq, hkv, gpu_device):
 def test_long_chunk_without_split_workspace(gpu_device):
     """A plan whose workspace does not hold the long-chunk kernel's split states
     is accepted and runs the kernel that needs none."""
-    import ctypes
-    from llm_gpu_kernels_amd import _native as N
     q, segs = _values(9, 500, (8192, 2049, 575), gpu_device)
     plan = prepare_segmented_gqa(q, segs)
     assert plan.splits_workspace_bytes > 0

@@ -142,6 +142,36 @@ def test_layout_rejects_invalid_descriptors(kw):
     assert N.last_error()
 
 
+def _gqa_choice(tokens, history, hq, hkv, cus=256):
+    d = N.GqaDesc()
+    d.T, d.Hq, d.Hkv, d.D, d.num_segments = tokens, hq, hkv, 128, len(history) + 1
+    for i, length in enumerate((*history, tokens)):
+        d.len[i], d.k[i], d.v[i] = length, 1 << 20, 1 << 20
+        d.k_stride[i] = d.v_stride[i] = hkv * 128
+    d.q = d.out = 1 << 20
+    out = (ctypes.c_int32 * 2)()
+    assert N.lib().gqa_seg_choice(ctypes.byref(d), cus, out) == 0, N.last_error()
+    return tuple(out)
+
+
+def test_long_chunk_attention_choice():
+    """The long-chunk kernel where it measured faster (tokens x history keys, query /
+    KV heads), the short-chunk kernel where that one did: few stages, and splits
+    whose further rounds cost more than they save."""
+    short, long_, mid, most = (16, 0, 1), (8192, 2049, 575), (1024, 512, 256), (4000, 64, 32)
+    for hq, hkv in ((32, 8), (16, 8), (8, 8), (64, 8), (8, 1), (4, 4)):
+        for tokens in (1, 32, 255):
+            assert _gqa_choice(tokens, long_, hq, hkv)[0] == 0
+        for history in ((), (1,), short, (100, 50, 50), (500, 0, 0)):
+            assert _gqa_choice(256, history, hq, hkv)[0] == 0, (hq, hkv, history)
+    assert _gqa_choice(512, mid, 32, 8)[0] == _gqa_choice(1024, mid, 32, 8)[0] == 0
+    assert _gqa_choice(3000, short, 16, 8)[0] == _gqa_choice(3000, (300, 0, 7), 8, 8)[0] == 0
+    assert _gqa_choice(4096, (500, 0, 0), 4, 4) == (1, 4)
+    assert _gqa_choice(2048, short, 32, 8) == _gqa_choice(2048, long_, 32, 8) == (1, 1)
+    assert _gqa_choice(1024, long_, 32, 8) == (1, 2) and _gqa_choice(512, long_, 32, 8) == (1, 4)
+    assert _gqa_choice(2048, long_, 16, 8) == (1, 2) and _gqa_choice(1024, short, 64, 8) == (1, 1)
+
+
 def test_plan_create_rejects_null_pointers():
     d = _desc()
     handle = ctypes.c_void_p()
