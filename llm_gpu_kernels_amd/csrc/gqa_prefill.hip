@@ -179,6 +179,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_kernel(GqaArgs a, int nq
         const uint32_t b = (uint32_t)(lw * 4 + j);
         buffer_load_lds16(vrs, buf + kVTile + b * kVBlock, (b + 16u * kr) * vsb + (uint32_t)((lane & 15) << 4));
       }
+      asm volatile("" ::: "memory");  // the counted waits below rely on the stages' order
       slot = slot == kSlots - 1 ? 0 : slot + 1;
     };
     for (int st = 0; st < kSlots - 1 && st < nst; ++st) issue(st);

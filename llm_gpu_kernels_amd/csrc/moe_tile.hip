@@ -123,6 +123,11 @@ __device__ __forceinline__ void buffer_load_lds16(__amdgpu_buffer_rsrc_t rs, uin
 #endif
 }
 
+// Ends a group of loads.  A counted wait is right only while the groups are
+// issued in program order; loads with an LDS destination and loads into
+// registers do not alias, so without this the scheduler may swap them.
+__device__ __forceinline__ void order_loads() { asm volatile("" ::: "memory"); }
+
 __device__ __forceinline__ int sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // The unit sequence, held by every wave: lane l has the row counts and first
@@ -310,6 +315,7 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
       if (b >= nb) break;
       buffer_load_lds16(brs, buf + kABytes + (b * 32 + lw * 8) * 128, boff[b] | ob, koff);
     }
+    order_loads();
     slot = slot == kSlots - 1 ? 0 : slot + 1;
     if (++kt_next == KT) {
       kt_next = 0;
@@ -385,6 +391,7 @@ __device__ __forceinline__ void load_role_w4(const ExpertArgs &a, const UnitMap 
     uint8_t *dst = smem + R::kB0 + b_slot * R::kBStride + lw * 8 * 128;
 #pragma unroll
     for (int b = 0; b < NBM; ++b) buffer_load_lds16(brs, dst + b * 32 * 128, boff[b], (uint32_t)b_kt * (kBK * 2));
+    order_loads();
     b_slot = b_slot == R::kBSlots - 1 ? 0 : b_slot + 1;
     if (++b_kt == KT) {
       b_kt = 0;
@@ -417,6 +424,7 @@ __device__ __forceinline__ void load_role_w4(const ExpertArgs &a, const UnitMap 
           u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, woff + (uint32_t)(j * KP) * 1024u, w_kp * 1024, 0));
       sc[buf][j] = __builtin_amdgcn_raw_buffer_load_b16(srs, soff + (uint32_t)(j * KP) * 32u, w_kp * 32, 0);
     }
+    order_loads();
     if (++w_kp == KP) {
       w_kp = 0;
       ++w_unit;
