@@ -7,6 +7,7 @@ reference's functional specs (N(0,1) weights) use the reference's own
 0.008/0.008 limits against the FP32 oracle plus a tight check against the
 rounding-staged oracle.
 """
+import ctypes
 import json
 from pathlib import Path
 
@@ -16,6 +17,7 @@ import torch
 from llm_gpu_kernels_amd import (GemmConfig, dequantize_tiled, prepare_moe, prepare_routed_moe,
                                  prepare_w4_layout_moe, repack_gate_up,
                                  prepare_w4_moe, quantize_gate_up, tile_gate_up)
+from llm_gpu_kernels_amd import _native as N
 from llm_gpu_kernels_amd.workloads import make_layer
 from oracle import moe_oracle as O
 
@@ -120,21 +122,38 @@ def _ids_with_counts(counts, tokens, k):
     return flat.view(k, tokens).t().contiguous().to(torch.int32)
 
 
-@pytest.mark.parametrize("hidden,inter,w4,special", [
-    (2048, 768, False, [160, 161, 320, 321, 1, 31, 33, 159]),  # units of 96 rows (gate/up) and 160 (down)
-    (2080, 800, False, [128, 129, 64, 65, 97, 32, 480, 2]),    # half stages at the end of K, partial weight tiles
-    (1056, 96, False, [300, 1, 0, 0, 161, 0, 96, 5]),          # I below one weight tile and one and a half stages
-    (512, 256, False, [40, 33, 64, 32, 1, 0, 31, 48]),         # 32-row units, four ring slots
-    (2048, 768, True, [160, 161, 320, 321, 1, 31, 33, 159]),   # W4: 96-row units
-    (1152, 2080, True, [128, 129, 64, 65, 97, 32, 480, 2]),    # 160-row units, nine word pairs, partial tiles
-    (128, 512, True, [300, 1, 0, 0, 161, 0, 96, 5]),           # 32-row units of one word pair (two stages)
+def _kernels(plan):
+    """(gate/up kernel, its rows per unit, down kernel, its rows) of a plan's shape."""
+    out = (ctypes.c_int32 * 4)()
+    cus = torch.cuda.get_device_properties(plan.x.device).multi_processor_count
+    N.check(N.lib().moe_gemm_choice(ctypes.byref(plan._desc), cus, out), "choice")
+    return tuple(out)
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,w4,special,rows", [
+    # bf16, three ring slots: units of up to 96, 128 and 160 rows
+    (512, 2048, 768, False, [96, 97, 192, 193, 1, 31, 33, 161], (96, 96)),
+    (520, 2048, 768, False, [128, 129, 256, 257, 1, 31, 97, 2], (128, 128)),
+    (660, 2080, 800, False, [160, 161, 320, 321, 480, 2, 33, 159], (160, 160)),  # half stages, partial weight tiles
+    (512, 1056, 96, False, [300, 1, 0, 0, 161, 0, 96, 5], (32, 96)),  # I below one weight tile and 1.5 stages
+    # four slots: 64 and 32 rows
+    (300, 2048, 768, False, [64, 65, 128, 129, 1, 31, 33, 96], (64, 64)),
+    (512, 512, 256, False, [40, 33, 64, 32, 1, 0, 31, 48], (32, 32)),
+    # W4: eight token slots of 96 rows (also one word pair, two stages), of 64 and of 32, four of 128 and 160
+    (512, 2048, 768, True, [96, 97, 192, 193, 1, 31, 33, 161], (96, 96)),
+    (512, 128, 640, True, [96, 97, 192, 193, 1, 31, 33, 161], (96, 32)),
+    (300, 2048, 768, True, [64, 65, 128, 129, 1, 31, 33, 96], (64, 64)),
+    (512, 384, 256, True, [40, 33, 64, 32, 1, 0, 31, 48], (32, 32)),
+    (520, 128, 768, True, [300, 1, 0, 0, 161, 0, 129, 5], (128, 32)),
+    (512, 1152, 2080, True, [160, 161, 320, 321, 1, 31, 33, 159], (160, 96)),  # nine word pairs, partial tiles
 ])
-def test_tiled_row_blocks(hidden, inter, w4, special, gpu_device):
+def test_tiled_row_blocks(tokens, hidden, inter, w4, special, rows, gpu_device):
     """The LDS-tiled kernels cut each expert's rows into equal blocks of at most
-    160, 96, 64 or 32: row counts around those edges (and experts without rows),
-    weight tiles and K stages that end inside the matrices.  Each grouped row
-    is checked against the FP32 oracle, and a second run is bitwise equal."""
-    tokens, k, e = 512, 4, 16
+    160, 128, 96, 64 or 32 (asserted): row counts around those edges (and experts
+    without rows), weight tiles and K stages that end inside the matrices.  Each
+    grouped row is checked against the FP32 oracle, and a second run is bitwise
+    equal."""
+    k, e = 4, 16
     rest = tokens * k - sum(special)
     counts = special + [rest // 8 + (1 if i < rest % 8 else 0) for i in range(8)]
     ids = _ids_with_counts(counts, tokens, k)
@@ -148,6 +167,7 @@ def test_tiled_row_blocks(hidden, inter, w4, special, gpu_device):
         gu = O.dequantize_w4(packed.words, packed.scales)
     else:
         plan = prepare_moe(xd, *_to(gpu_device, gu), dnd, idd, wd, config=GemmConfig(block_m=64))
+    assert _kernels(plan) == (N.GEMM_TILED, rows[0], N.GEMM_TILED, rows[1])
     first = plan.run().clone()
     out = plan.run()
     torch.cuda.synchronize()
@@ -183,23 +203,25 @@ def test_tiled_swiglu_matches_streaming(gpu_device):
     assert ((act.double() - exact).abs() <= exact.abs() * 2.0 ** -8 + 2e-36).all()
 
 
-@pytest.mark.parametrize("tokens,experts,hidden,inter,topk", [
-    (192, 64, 1024, 512, 4),   # 12 rows per expert, 256 down tiles: streaming gate/up, tiled down
-    (272, 64, 512, 512, 4),    # 17 rows: gate/up tiled (256 tiles), streaming down (128 tiles)
-    (324, 64, 512, 512, 4),    # 20.25 rows: both tiled
-    (100, 32, 2880, 1440, 4),  # run-time-K shape, 32-row tasks, both tiled
-    (17, 32, 2880, 1440, 4),   # about two rows: gate/up tiled, down run-time-K
-    (24, 32, 2048, 1440, 4),   # rows a multiple of 4 KiB apart: run-time-K gate/up
+@pytest.mark.parametrize("tokens,experts,hidden,inter,topk,gate_up,down", [
+    (188, 64, 1024, 512, 4, N.GEMM_LDS_STREAM, N.GEMM_LDS_STREAM),  # 11.75 rows per expert
+    (192, 64, 1024, 512, 4, N.GEMM_LDS_STREAM, N.GEMM_TILED),       # 12 rows, 256 down tiles
+    (272, 64, 512, 512, 4, N.GEMM_TILED, N.GEMM_STREAM),            # 17 rows, 256 gate/up tiles and 128 down tiles
+    (324, 64, 512, 512, 4, N.GEMM_TILED, N.GEMM_TILED),             # 20.25 rows
+    (100, 32, 2880, 1440, 4, N.GEMM_TILED, N.GEMM_TILED),           # run-time-K shape, 32-row tasks
+    (17, 32, 2880, 1440, 4, N.GEMM_TILED, N.GEMM_RUNTIME_K),        # about two rows
+    (24, 32, 2048, 1440, 4, N.GEMM_RUNTIME_K, N.GEMM_RUNTIME_K),    # weight rows a multiple of 4 KiB apart
 ])
-def test_tiled_rules_below_64_rows(tokens, experts, hidden, inter, topk, gpu_device):
+def test_tiled_rules_below_64_rows(tokens, experts, hidden, inter, topk, gate_up, down, gpu_device):
     """Shapes on both sides of the rules that take 16- and 32-row tasks to the
-    LDS-tiled kernels, through the router, against the FP32 oracle."""
+    LDS-tiled kernels (asserted), through the router, against the FP32 oracle."""
     x, gu, dn, _, _ = O.make_inputs(tokens=tokens, experts=experts, topk=topk, hidden=hidden, intermediate=inter,
                                     id_dtype=torch.int32, pattern="random", seed=tokens + hidden)
     logits = torch.randn((tokens, experts), generator=torch.Generator().manual_seed(tokens))
     logits[:, 0] += 2.0  # a hot expert: several row blocks
     xd, gud, dnd, ld = _to(gpu_device, x, gu, dn, logits)
     plan = prepare_routed_moe(xd, ld, gud, dnd, topk)
+    assert _kernels(plan)[::2] == (gate_up, down)
     out = plan.forward(xd, ld)
     torch.cuda.synchronize()
     plan.check_inputs()
