@@ -198,17 +198,36 @@ static bool tiled_down(const ExpertArgs &a, int token_block, int path, int num_c
 // K = 8): T = 600 88 / 91 us, T = 1024 112 / 114, T = 1536 136 / 143 (Zipf 156 /
 // 150), T = 2048 179 / 143, T = 4096 311 / 233; with few experts the pair
 // kernel's workgroups (16 column blocks of one task) do not fill the CUs: E =
-// 16, 64 rows each 41 / 30 us.
+// 16, 64 rows each 41 / 30 us.  Layers at other I: I = 96, T = 512 / 1024 / 1536 61 /
+// 67, 72 / 77 and 85 / 91 us; I = 192 level; I = 384, T = 512 103 / 117, but T = 1024
+// 148 / 133.
 static bool w4_pair_preferred(const ExpertArgs &a, int num_cus) {
   return a.H == 2048 && (long long)a.R < 128LL * a.E && (long long)a.E * ((a.I + 255) / 256) * 4 >= num_cus;
 }
 
+// W4 gate/up of 64-row tasks at other H: the kernel of one unit per wave decodes
+// once per task and keeps every CU's waves busy where the tiled kernel has few or
+// short units.  Measured, layer, this kernel against tiled (K = 4): E = 64, H =
+// 512, I = 480, 160 rows each 56 / 67 us; H = 1024, I = 96, 160 rows 49 / 58; E = 8,
+// H = 256, I = 256, 64 rows 25 / 29; at 32 rows each E = 64, H = 1536, I = 768 83 /
+// 94 and H = 3072 133 / 150, E = 32, H = 4096, I = 1536 163 / 188.  With larger
+// matrices and more rows the tiled kernel: E = 64, H = 1024, I = 512, 64 / 256 rows
+// 62 / 59 and 113 / 107 (96 rows 70 / 79), H = 1792 87 / 79 and 180 / 162, E = 32, H
+// = 2560, I = 1024, 64 / 128 rows 111 / 100 and 151 / 122.  (One 32-column block of
+// H = 1792: the run-time-K kernel, E = 8 35 / 27 us.)
+static bool w4_wave_preferred(const ExpertArgs &a) {
+  const long long hi = (long long)a.H * a.I;
+  if (a.H == 2048 || !wave_w4_shape_ok(a.H, a.I, 64) || (hi < 65536 && a.H > 1536)) return false;
+  return hi < (1 << 19) || (long long)a.R < 48LL * a.E;
+}
+
 GemmKernel gate_up_kernel(const ExpertArgs &a, int token_block, bool w4, int path, int num_cus) {
-  // W4 with several rows per expert, and every 64-row task: decode each weight
-  // fragment once for up to 64 token rows (one unit per wave).  With about one
-  // row per expert the split-K streaming kernel overlaps the decode better, and
-  // with the folded decode it is faster for 16-row tasks too (T = 193: gate/up
-  // 49 vs 61 us).
+  // W4: 64-row tasks by the three rules above.  Several rows per expert in
+  // shorter tasks: decode each weight fragment once for the task (one unit per
+  // wave).  With about one row per expert the split-K streaming kernel overlaps
+  // the decode better, and with the folded decode it is faster for 16-row tasks
+  // too (T = 193: gate/up 49 vs 61 us).
+  if (w4 && token_block == 64 && w4_wave_preferred(a)) return kWaveGemm;
   if (w4 && token_block == 64 && !w4_pair_preferred(a, num_cus) && tiled_gate_up(a, token_block, path, num_cus))
     return kTileGemm;
   const bool wave_ok = w4 && (token_block != 64 || a.H == 2048) && wave_w4_shape_ok(a.H, a.I, token_block);

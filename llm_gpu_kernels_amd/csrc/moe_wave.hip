@@ -451,7 +451,8 @@ hipError_t launch_wave_w4_gate_up(const ExpertArgs &a, int task_capacity, int to
   switch (token_block) {
     case 16: return launch_mt<1>(a, task_capacity, s);
     case 32: return launch_mt<2>(a, task_capacity, s);
-    default: return hipErrorInvalidValue;  // 64-row tasks: the pair kernel or the tiled one
+    case 64: return launch_mt<4>(a, task_capacity, s);
+    default: return hipErrorInvalidValue;
   }
 }
 

@@ -118,7 +118,7 @@ def test_tiled_units_fill_idle_cus(experts, fmt):
         return experts * (-(-inter // 128)) * (-(-mean // rows))
     for inter in (96, 256, 512, 768, 1536):
         for mean in list(range(100, 170)) + [192, 256, 320, 321]:
-            kernel, rows, _, _ = _choice(T=mean * experts, K=1, E=experts, H=1024, I=inter, fmt=fmt, tb=64)
+            kernel, rows, _, _ = _choice(T=mean * experts, K=1, E=experts, H=1152, I=inter, fmt=fmt, tb=64)
             assert kernel == N.GEMM_TILED and rows in (32, 64, 96, 128, 160)
             n = units(inter, mean, rows)
             assert 2 * n >= 256 or n == units(inter, mean, 32), (inter, mean, rows)
@@ -140,6 +140,22 @@ def test_layout_rejects_invalid_descriptors(kw):
     rc, _ = _layout(_desc(**kw))
     assert rc == N.MOE_EINVAL
     assert N.last_error()
+
+
+@pytest.mark.parametrize("tokens,experts,hidden,inter,kernel", [
+    (256, 8, 256, 96, N.GEMM_DECODE_ONCE), (256, 8, 512, 96, N.GEMM_DECODE_ONCE),  # small matrices
+    (2560, 64, 512, 480, N.GEMM_DECODE_ONCE), (2560, 64, 1024, 96, N.GEMM_DECODE_ONCE),
+    (512, 64, 1536, 768, N.GEMM_DECODE_ONCE), (767, 64, 1536, 768, N.GEMM_DECODE_ONCE),  # below 48 rows per expert
+    (768, 64, 1536, 768, N.GEMM_TILED), (1024, 32, 2560, 1024, N.GEMM_TILED), (1024, 64, 1024, 512, N.GEMM_TILED),
+    (256, 8, 1792, 32, N.GEMM_RUNTIME_K), (256, 8, 128, 512, N.GEMM_TILED), (256, 8, 384, 96, N.GEMM_RUNTIME_K),
+    (1024, 64, 2048, 768, N.GEMM_DECODE_ONCE), (2048, 64, 2048, 768, N.GEMM_TILED),  # H = 2048: the pair kernel
+])
+def test_w4_64_row_choice(tokens, experts, hidden, inter, kernel):
+    """The gate/up kernel of W4 64-row tasks (K = 4): each where it measured
+    fastest of decode-once, tiled and run-time-K."""
+    kw = dict(T=tokens, E=experts, H=hidden, I=inter, K=4, fmt=N.WEIGHTS_W4G128)
+    assert _layout(_desc(**kw))[1].token_block == 64
+    assert _choice(**kw)[0] == kernel
 
 
 def _gqa_choice(tokens, history, hq, hkv, cus=256):

@@ -411,6 +411,8 @@ FLEX_SHAPES = [
     (9, 8, 2, 1152, 384, True),      # W4 run-time-K gate/up, 16-row tasks
     (100, 8, 2, 1152, 384, True),    # 32-row tasks
     (300, 8, 2, 1152, 384, True),    # 64-row tasks
+    (300, 8, 2, 512, 96, True),      # 64-row tasks in the W4 wave kernel, six of eight waves with columns
+    (150, 8, 2, 1024, 544, True),    # the same, below 48 rows per expert, 34 column blocks
     # K <= 256: the waves split the columns instead of K (gate/up at H = 256,
     # down at I = 96: one GPU's share of the Qwen layer under 8-way tensor parallelism)
     (100, 8, 2, 256, 96, False),     # 32-row tasks, both GEMMs column-split
