@@ -67,7 +67,7 @@ int choose_token_block(const moe_desc *d) {
 int choose_path(const moe_desc *d, int tb) {
   const bool w4 = is_w4(d->weight_format);
   if (tb == 64) {
-    if (moe::tile_shape_ok(d->H, d->I, w4)) return moe::kTile;
+    if (moe::tile_shape_ok(d->H, d->I)) return moe::kTile;
     return moe::stream_shape_ok(d->H, d->I, w4) ? moe::kStream : moe::kGeneric;
   }
   return moe::stream_shape_ok(d->H, d->I, w4) ? moe::kStream : moe::kGeneric;

@@ -99,7 +99,7 @@ bool tile_gemm_ok(int H, int I);
 // Token rows of a unit at most.
 int tile_unit_rows(const ExpertArgs &a, bool down, int num_cus);
 // Shapes that report the tiled family (moe_layout.fast_path 2).
-bool tile_shape_ok(int H, int I, bool w4);
+bool tile_shape_ok(int H, int I);
 
 // Expert-stage kernel families (moe_layout.fast_path).
 // kGeneric: the run-time-K MFMA kernels, with 64-row tasks the tiled bf16

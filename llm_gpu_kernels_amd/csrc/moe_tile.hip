@@ -738,14 +738,16 @@ hipError_t launch_tile(const ExpertArgs &a, int num_cus, hipStream_t s) {
 
 bool tile_gemm_ok(int H, int I) {
   // Whole 32-row fragments and 16-byte chunks; byte offsets within one
-  // expert's matrix, overshoot of the last tile included, fit 32 bits.
-  return H % 32 == 0 && I % 32 == 0 && (long long)H * I * 2 < (1LL << 31);
+  // expert's gate, up or down matrix, the last tile's rows past its end
+  // included (they must not wrap back into it), fit 32 bits.  (Descriptors of a
+  // wave's own 64 rows instead of the matrix would take larger ones, but
+  // lengthen the loaders' set-up per unit: T = 4096 442 -> 453 us, W4 T = 3001 391
+  // -> 419, E = 128, H = 2048, I = 768, K = 8.)
+  const long long limit = 1LL << 32;
+  return H % 32 == 0 && I % 32 == 0 && 2LL * H * (I + kBN / 2) < limit && 2LL * I * (H + kBN) < limit;
 }
 
-bool tile_shape_ok(int H, int I, bool w4) {
-  if (I % 128 || H % 256 || !tile_gemm_ok(H, I)) return false;
-  return w4 ? wave_w4_shape_ok(H, I, 64) : true;  // W4 gate/up runs in the wave kernel
-}
+bool tile_shape_ok(int H, int I) { return I % 128 == 0 && H % 256 == 0 && tile_gemm_ok(H, I); }
 
 int tile_unit_rows(const ExpertArgs &a, bool down, int num_cus) { return 32 * unit_blocks(a, down, num_cus); }
 

@@ -142,6 +142,16 @@ def test_layout_rejects_invalid_descriptors(kw):
     assert N.last_error()
 
 
+def test_tiled_matrix_size():
+    """The tiled kernels take matrices whose byte offsets, the rows of the last tile
+    past the end included, fit 32 bits: neither smaller ones are refused nor do
+    long rows wrap."""
+    for h, i in ((32768, 32768), (34816, 32800), (65024, 32768), (32768, 65024)):
+        assert _choice(T=40, E=1, K=1, H=h, I=i)[::2] == [N.GEMM_TILED, N.GEMM_TILED], (h, i)
+    for h, i in ((65536, 32768), (1 << 24, 32), (32, 1 << 23)):  # 127 rows of 32 MiB, 255 of 16 MiB
+        assert _choice(T=40, E=1, K=1, H=h, I=i)[::2] == [N.GEMM_RUNTIME_K, N.GEMM_RUNTIME_K], (h, i)
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,inter,kernel", [
     (256, 8, 256, 96, N.GEMM_DECODE_ONCE), (256, 8, 512, 96, N.GEMM_DECODE_ONCE),  # small matrices
     (2560, 64, 512, 480, N.GEMM_DECODE_ONCE), (2560, 64, 1024, 96, N.GEMM_DECODE_ONCE),

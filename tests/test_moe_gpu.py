@@ -178,6 +178,32 @@ def test_tiled_row_blocks(tokens, hidden, inter, w4, special, rows, gpu_device):
     assert m["passed"], m
 
 
+@pytest.mark.parametrize("hidden,inter", [(32768, 34816), (34816, 32800)])
+def test_tiled_matrices_over_2_gib(hidden, inter, gpu_device):
+    """Expert matrices whose byte offsets need the 32nd bit, against fp32 products
+    of column blocks; the last gate/up tile of the second ends a quarter full."""
+    tokens = 64
+    gen = torch.Generator(device=gpu_device).manual_seed(hidden)
+    gu = torch.empty((1, 2 * inter, hidden), dtype=torch.bfloat16, device=gpu_device)
+    dn = torch.empty((1, hidden, inter), dtype=torch.bfloat16, device=gpu_device)
+    assert dn.numel() * 2 > 1 << 31
+    for t in (gu, dn):
+        t.normal_(0.0, 0.02, generator=gen)
+    x = torch.randn((tokens, hidden), generator=gen, device=gpu_device).to(torch.bfloat16)
+    ids = torch.zeros((tokens, 1), dtype=torch.int32, device=gpu_device)
+    plan = prepare_moe(x, gu, dn, ids, torch.ones((tokens, 1), device=gpu_device))
+    assert _kernels(plan)[::2] == (N.GEMM_TILED, N.GEMM_TILED)
+    out = plan.run().float()
+
+    def product(a, w):
+        return torch.cat([a.float() @ part.float().t() for part in w.split(2048)], dim=1)
+
+    h = product(x, gu[0]).to(torch.bfloat16).float()
+    act = (torch.nn.functional.silu(h[:, :inter]) * h[:, inter:]).to(torch.bfloat16)
+    m = O.error(out.cpu(), product(act, dn[0]).cpu())
+    assert m["passed"], m
+
+
 def test_tiled_swiglu_matches_streaming(gpu_device):
     """One-hot token rows make gate and up exact, so the activations of the tiled
     kernels are bit for bit those of the streaming kernels, over every sign and
