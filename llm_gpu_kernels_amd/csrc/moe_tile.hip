@@ -696,28 +696,34 @@ hipError_t launch_nbm(const ExpertArgs &a, int max_rows, int num_cus, hipStream_
 // 334 us per layer at E = 128, H = 2048, I = 768, K = 8, T = 2048 (mean 128)
 // and 425 vs 448 at E = 32, H = I = 2880, K = 4, T = 1024 (Zipf routing).
 // Below a mean of 128 rows 96-row units waste less of the last round: T = 1024
-// Zipf 242 vs 255 us, uniform 266 vs 267 (64-row units: 262 and 293).  Where the
-// units of the mean expert leave half the CUs idle, lower ones that make more
-// of them: the four-slot ring of 64 rows (16 experts, H = 2048, I = 768, 64
-// rows each: 66.3 vs 67.9 us; 88 rows 71.3 -> 67.6 for the down projection), 96
-// instead of 160 rows where one block holds the whole expert (128 rows each:
-// 82.2 -> 73.1 us), then 32-row units where an expert's rows still make more of
-// them (E = 8, H = 512, I = 256, 256 rows each: 26.5 vs 28.3 us).  Two 64-row
-// blocks also where they leave a quarter of one round for the experts above
-// the mean (16 experts of 100 / 127 rows, gate/up: 75.5 -> 70.5 / 73.5 -> 71.9 us;
-// with less to spare they start a second round: down at 127 rows 73.5 -> 80.9).
+// Zipf 242 vs 255 us, uniform 266 vs 267 (64-row units: 262 and 293).  While
+// the units leave half the CUs idle, lower ones that make more of them: the
+// four-slot ring of 64 rows (16 experts, H = 2048, I = 768, 64 rows each: 66.3 vs
+// 67.9 us), 96 rows where one 128- or 160-row block holds the mean expert (128
+// rows each, gate/up: 81.4 -> 74.3 us, Zipf 78.7 -> 74.9), then 32-row units where
+// an expert's rows still make more of them (E = 8, H = 512, I = 256, 256 rows
+// each: 26.5 vs 28.3 us).  Where they would then fill all the CUs, the experts
+// above the mean of a skewed routing make a second round (16 experts of 88 rows,
+// down with 64 rows: uniform 67.8 -> 65.8 us, Zipf 68.6 -> 75.3), so exactly half
+// is lowered only where three quarters result (E = 16, H = 1024, I = 512, 175 rows
+// each: 46.2 -> 37.7 us, Zipf 46.8 -> 37.8).  Two 64-row blocks instead of two in 96-row units under the
+// same condition: with a quarter of the round to spare up to 112 rows, with
+// half above (gate/up of 16 experts of 97 / 119 rows 74.3 -> 69.8 / 74.0 -> 75.0, Zipf
+// 73.6 -> 70.9 / 74.1 -> 72.2, of 127 rows Zipf 80.9 -> 95.4; H = 1024, I = 512, 128
+// rows 39.7 -> 36.7).
 int unit_blocks(long long R, int E, int ntiles, int num_cus) {
   const long long mean = (R + E - 1) / E;
   auto units = [&](int nb) { return (long long)E * ntiles * ((mean + 32 * nb - 1) / (32 * nb)); };
   int nb = mean >= 128 ? kMaxNB : mean > 40 ? 3 : 2;
   if (nb == 3 && mean <= 64 && 2 * units(2) <= num_cus) nb = 2;
-  if (nb == 3 && mean > 96 && 4 * units(2) <= 3LL * num_cus) nb = 2;
   while (2 * units(nb) <= num_cus) {
     int n = nb - 1;
     while (n > 1 && units(n) == units(nb)) --n;  // the next height that makes more units
-    if (n < 1 || (n == 1 && (mean <= 64 || 2 * units(nb) == num_cus))) break;
+    if (n < 1 || (n == 1 && mean <= 64)) break;
+    if (2 * units(nb) == num_cus && 4 * units(n) > 3LL * num_cus) break;
     nb = n;
   }
+  if (nb == 3 && mean > 96 && mean <= 128 && 4 * units(2) <= (mean <= 112 ? 3LL : 2LL) * num_cus) nb = 2;
   return nb;
 }
 

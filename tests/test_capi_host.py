@@ -117,15 +117,17 @@ def test_tiled_units_fill_idle_cus(experts, fmt):
     def units(inter, mean, rows):
         return experts * (-(-inter // 128)) * (-(-mean // rows))
     for inter in (96, 256, 512, 768, 1536):
-        for mean in list(range(100, 170)) + [192, 256, 320, 321]:
+        for mean in list(range(97, 170)) + [192, 256, 320, 321]:
             kernel, rows, _, _ = _choice(T=mean * experts, K=1, E=experts, H=1152, I=inter, fmt=fmt, tb=64)
             assert kernel == N.GEMM_TILED and rows in (32, 64, 96, 128, 160)
             n = units(inter, mean, rows)
             assert 2 * n >= 256 or n == units(inter, mean, 32), (inter, mean, rows)
     # 16 experts, gate/up and down (six and eight weight tiles).
-    rows = {t: _choice(T=t, K=1, E=16, fmt=fmt)[1::2] for t in (1024, 1400, 1600, 2032, 2048, 2049, 4096)}
-    assert rows == {1024: [64, 64], 1400: [64, 64], 1600: [64, 96], 2032: [64, 96], 2048: [96, 96],
-                    2049: [128, 128], 4096: [160, 160]}
+    rows = {t: _choice(T=t, K=1, E=16, fmt=fmt)[1::2] for t in (1024, 1400, 1600, 1800, 2032, 2048, 2049, 4096)}
+    assert rows == {1024: [64, 64], 1400: [64, 96], 1600: [64, 96], 1800: [96, 96], 2032: [96, 96],
+                    2048: [96, 160], 2049: [128, 160], 4096: [160, 160]}
+    shape = dict(K=4, E=16, H=1152, I=512, fmt=fmt, tb=64)  # four gate/up tiles: half of the CUs, or three quarters
+    assert [_choice(T=t, **shape)[1] for t in (400, 500, 512, 600, 700)] == [64] * 5
     assert _choice(T=2048, fmt=fmt)[1] == 160  # every CU has units: the fewest weight reads
 
 

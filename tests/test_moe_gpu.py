@@ -132,17 +132,17 @@ def _kernels(plan):
 
 @pytest.mark.parametrize("tokens,hidden,inter,w4,special,rows", [
     # bf16, three ring slots: units of up to 96, 128 and 160 rows
-    (512, 2048, 768, False, [96, 97, 192, 193, 1, 31, 33, 161], (96, 96)),
-    (520, 2048, 768, False, [128, 129, 256, 257, 1, 31, 97, 2], (128, 128)),
+    (512, 2048, 768, False, [96, 97, 192, 193, 1, 31, 160, 161], (96, 160)),
+    (520, 2048, 768, False, [128, 129, 256, 257, 1, 31, 160, 161], (128, 160)),
     (660, 2080, 800, False, [160, 161, 320, 321, 480, 2, 33, 159], (160, 160)),  # half stages, partial weight tiles
     (512, 1056, 96, False, [300, 1, 0, 0, 161, 0, 96, 5], (32, 96)),  # I below one weight tile and 1.5 stages
     # four slots: 64 and 32 rows
-    (300, 2048, 768, False, [64, 65, 128, 129, 1, 31, 33, 96], (64, 64)),
+    (300, 2048, 768, False, [64, 65, 128, 129, 1, 31, 33, 97], (64, 96)),
     (512, 512, 256, False, [40, 33, 64, 32, 1, 0, 31, 48], (32, 32)),
     # W4: eight token slots of 96 rows (also one word pair, two stages), of 64 and of 32, four of 128 and 160
-    (512, 2048, 768, True, [96, 97, 192, 193, 1, 31, 33, 161], (96, 96)),
+    (512, 2048, 768, True, [96, 97, 192, 193, 1, 31, 33, 161], (96, 160)),
     (512, 128, 640, True, [96, 97, 192, 193, 1, 31, 33, 161], (96, 32)),
-    (300, 2048, 768, True, [64, 65, 128, 129, 1, 31, 33, 96], (64, 64)),
+    (300, 2048, 768, True, [64, 65, 128, 129, 1, 31, 33, 96], (64, 96)),
     (512, 384, 256, True, [40, 33, 64, 32, 1, 0, 31, 48], (32, 32)),
     (520, 128, 768, True, [300, 1, 0, 0, 161, 0, 129, 5], (128, 32)),
     (512, 1152, 2080, True, [160, 161, 320, 321, 1, 31, 33, 159], (160, 96)),  # nine word pairs, partial tiles
