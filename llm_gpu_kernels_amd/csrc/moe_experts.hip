@@ -162,8 +162,9 @@ constexpr bool kDmaDown = true;
 //    8): T = 300 282 / 256, T = 400 297 / 257, Zipf 288 / 190, T = 500 351 / 260 (a
 //    hot expert's weights are streamed once per 32-row task); at 16 and below the
 //    LDS-streaming gate/up reads weights faster (T = 193: 137 / 160 us), but the
-//    down projection is level from 12 rows on (77 / 77) and far better under
-//    skewed routing (Zipf 56 / 46).  16 experts (96 gate/up tiles): 51 / 58 at 16
+//    down projection is level from 12 rows on (77 / 77; layers at T = 200 / 224 /
+//    256 229.5 / 227.6, 239.3 / 234.4 and 263.9 / 253.1) and far better under skewed
+//    routing (56 / 46; layers 185 / 174, 200 / 184 and 213 / 193).  16 experts (96 gate/up tiles): 51 / 58 at 16
 //    rows, 58 / 59 at 19, 65 / 61 at 28.
 //  * run-time-K shapes of 64-row tasks: E = 32, H = I = 2880, T = 512 768 / 312;
 //    E = 128, H = 2048, I = 96, T = 1024 113 / 76; not for matrices so small that

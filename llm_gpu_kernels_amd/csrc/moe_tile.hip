@@ -352,7 +352,7 @@ __device__ __forceinline__ void lds_write_b128(uint32_t addr, u32x4 v) {
 
 // W4G128 gate/up: the loader waves stream the int4 words into registers (one
 // 1 KiB load per 16 rows x 128 K, i.e. per two stages, three pairs of stages ahead),
-// decode them bit-exactly and write the bf16 weight tile of stage st + 2 while
+// decode them bit-exactly and write the bf16 weight tile of stage st + 1 while
 // the MFMA waves multiply stage st, so each weight is decoded once per unit of
 // up to 160 rows and the MFMA waves issue no decode.  Token tiles come as in
 // the bf16 kernel, always NBM loads per stage (blocks past the unit's rows are

@@ -223,11 +223,11 @@ hipError_t launch_mt(const ExpertArgs &a, int task_capacity, hipStream_t s) {
 // (rows 16-31), so the MFMA output puts gate and up of a (feature, token) in
 // the same lane (output rows 8q + 4h + i: q = 0, 1 gate, q = 2, 3 up).
 //
-// Launched for 64-row tasks (MT = 3) and, with several rows per expert, for
-// 16-row tasks (MT = 1).  Unit = (pass, 16 intermediate columns).  A pass is
-// one planner task, or two consecutive tasks of an expert with at most 32*MT
-// rows together, so
-// each weight is decoded once for every row of such an expert.  Per 16-K step
+// Launched at H = 2048 for 64-row tasks below 128 rows per expert (MT = 3) and,
+// with several rows per expert, for 16-row tasks (MT = 1).  Unit = (pass, 16
+// intermediate columns).  A pass is one planner task, or two consecutive tasks
+// of an expert with at most 32*MT rows together, so each weight is decoded once
+// for every row of such an expert.  Per 16-K step
 // a wave decodes one packed int4 word per lane (w4_decode8, bit-exact with
 // the reference dequantisation) and multiplies it against up to MT 32-token
 // B fragments read from LDS.  The lane of a 32x32x16 A fragment holds row

@@ -400,9 +400,9 @@ def test_parallel_shard_shapes(shape, tokens, routing, w4, path, gpu_device):
 @pytest.mark.parametrize("tokens", [17, 193])
 def test_w4_token_blocks(tokens, gpu_device):
     """W4 gate/up with 16-, 32- and 64-row tasks: at T=17 the split-K streaming kernel
-    (16, 32 rows) and the one-unit-per-wave kernel (64 rows); at T=193 the wave kernel
-    with 1, 2 and 4 token blocks per fragment.  Each within tolerance of the FP32
-    oracle on the dequantised weights, and of the 16-row result."""
+    (16, 32 rows) and the pair kernel (64 rows); at T=193 the pair kernel (16, 64
+    rows) and the one-unit-per-wave kernel (32 rows).  Each within tolerance of the
+    FP32 oracle on the dequantised weights, and of the 16-row result."""
     lay = make_layer("qwen", tokens, seed=5, device=gpu_device)
     ids, w = O.route_topk(lay["logits"].cpu(), 8)
     packed = quantize_gate_up(lay["gate_up"].cpu())
@@ -414,6 +414,7 @@ def test_w4_token_blocks(tokens, gpu_device):
         plan = prepare_w4_moe(lay["x"], tiled, lay["down"], ids.to(gpu_device), w.to(gpu_device),
                               down_config=GemmConfig(block_m=bm))
         assert plan.layout.token_block == bm
+        assert _kernels(plan)[0] == (N.GEMM_STREAM if tokens == 17 and bm < 64 else N.GEMM_DECODE_ONCE)
         out = plan.run().clone()
         torch.cuda.synchronize()
         m = O.error(out, ref)
