@@ -209,10 +209,18 @@ __device__ __forceinline__ float swiglu(float g, float u) { return g / (1.0f + e
 __device__ __forceinline__ void store_row(uint16_t *p, u32x4 v) { __builtin_nontemporal_store(v, (u32x4 *)p); }
 
 // 16-byte chunk c of row m of a stage's 32-row fragment sits at chunk c ^
-// swz(m): the sixteen lanes of an operand read (consecutive rows, one chunk)
-// and of the W4 loaders' writes (rows 8 q + 4 hb + i, one chunk) each cover all
-// 64 banks.
-__device__ __forceinline__ int swz(int m) { return ((m >> 1) & 7) ^ ((m >> 3) & 2); }
+// swz(m).  A 128-byte row covers half of the 64 banks, so sixteen lanes served
+// together must hold each of the eight chunks twice, in an even and an odd row.
+// Those are lanes 0-3, 12-15, 20-23 and 24-27 of a 16-byte operand read (and the
+// other sixteen of 32), not consecutive ones: with (m >> 1) ^ (m >> 3 & 2), which
+// is conflict-free for consecutive lanes only, half of the LDS cycles were
+// conflicts (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE 0.50, now 0.02 in gate/up, 0.08
+// with the down epilogue, 0.30 with the W4 writes; times within 1 %: the LDS does
+// not bound these kernels).  The Gray code of m / 4 serves both groupings, in the operand reads
+// (consecutive rows, one chunk) and in the W4 loaders' writes (rows 8 q + 4 hb + i).
+__device__ __forceinline__ int swz(int m) { return (((m >> 2) ^ (m >> 3)) & 3) << 1 | ((m >> 1) & 1); }
+// swz(8 j + lr) for lr < 8 is (lr >> 1) ^ swz8(j).
+__device__ __forceinline__ uint32_t swz8(int j) { return (uint32_t)(4 * ((j ^ (j >> 1)) & 1) | 2 * (j & 1)); }
 
 // Weight row within a 32-row fragment that LDS row m of it holds: the MFMA
 // leaves output rows 8 q + 4 h + i (q, i = 0..3) in lane half h, so with this
@@ -268,7 +276,6 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
   const auto brs = __builtin_amdgcn_make_buffer_rsrc((void *)xbase, (short)0, (int)xbytes, 0x00020000);
   __amdgpu_buffer_rsrc_t ars;
   uint32_t aoff[kAPer], boff[NBM];
-  // Rows r = 8 j + lr: swz(r) = (lr / 2) ^ 4 (j & 1) ^ (j & 2).
   const uint32_t c0 = (uint32_t)((lane & 7) ^ (lr >> 1));
   int cur = -1, nb = 0;
   auto setup = [&](int i) {
@@ -283,7 +290,7 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
 #pragma unroll
     for (int j = 0; j < kAPer; ++j) {
       const int row = wrow0 + (j / 4) * 32 + frag_row((j & 3) * 8 + lr);
-      aoff[j] = (uint32_t)row * pitch + ((c0 ^ (4u * (j & 1)) ^ (j & 2u)) << 4);
+      aoff[j] = (uint32_t)row * pitch + ((c0 ^ swz8(j & 3)) << 4);
     }
     uint32_t rows[NBM];
     if (KIND == 0) token_rows<NBM>(a, un, lw, lr, rows);
@@ -291,7 +298,7 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
     for (int b = 0; b < NBM; ++b) {
       const int r0 = b * 32 + lw * 8 + lr;
       if (KIND == 1) rows[b] = (uint32_t)(un.row0 + (r0 < un.rows ? r0 : 0));
-      boff[b] = rows[b] * pitch + ((c0 ^ (4u * (lw & 1)) ^ (lw & 2u)) << 4);
+      boff[b] = rows[b] * pitch + ((c0 ^ swz8(lw)) << 4);
     }
   };
   int slot = 0, kt_next = 0, unit_next = 0;
@@ -304,12 +311,12 @@ __device__ __forceinline__ void load_role(const ExpertArgs &a, const UnitMap &ma
     uint8_t *buf = smem + slot * kSlotBytes;
     const uint32_t koff = (uint32_t)kt_next * (kBK * 2);
     const bool part = tail != 0 && kt_next == KT - 1;
-    const uint32_t oe = part && c0 >= tail ? 0xffffffffu : 0u;         // chunks past K: out of range
-    const uint32_t oo = part && (c0 ^ 4u) >= tail ? 0xffffffffu : 0u;  // (tail is 4: bit 1 of c plays no part)
+    // Chunks past K are out of range; tail is 4, so bit 2 of the chunk decides.
+    const uint32_t past[2] = {part && c0 >= tail ? 0xffffffffu : 0u, part && (c0 ^ 4u) >= tail ? 0xffffffffu : 0u};
 #pragma unroll
     for (int j = 0; j < kAPer; ++j)
-      buffer_load_lds16(ars, buf + (lw * 64 + j * 8) * 128, aoff[j] | (j & 1 ? oo : oe), koff);
-    const uint32_t ob = lw & 1 ? oo : oe;
+      buffer_load_lds16(ars, buf + (lw * 64 + j * 8) * 128, aoff[j] | past[swz8(j & 3) >> 2], koff);
+    const uint32_t ob = past[swz8(lw) >> 2];
 #pragma unroll
     for (int b = 0; b < NBM; ++b) {
       if (b >= nb) break;
