@@ -63,7 +63,8 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
 // Measured at E = 128, H = 2048, I = 768, K = 8 against 64-row tasks with 64 x
 // 32 wave tiles and every fragment of a stage read before its MFMAs: T = 4096
 // gate/up 350 -> 237 us, down 215 -> 146 us; T = 1024 Zipf 153 -> 137 and 92 ->
-// 80 us.  At T = 4096 the loads alone take 188 us (2.5 GB through L2, 966 MB of
+// 80 us (with a SwiGLU of hardware exponentials; swiglu below: + 15 us at T =
+// 4096).  At T = 4096 the loads alone take 188 us (2.5 GB through L2, 966 MB of
 // HBM reads, 5.1 TB/s), the MFMAs and LDS reads alone 111 us, the epilogues 27.
 constexpr int kBN = 256;                // weight rows per tile
 constexpr int kBK = 64;                 // K per stage: one 128-byte piece per row
@@ -366,7 +367,8 @@ __device__ __forceinline__ void lds_write_b128(uint32_t addr, u32x4 v) {
 // out of range), so every wait is a constant count.  T = 4096, E = 128, H =
 // 2048, I = 768, K = 8: 233 us (885 TFLOP/s) against 311 us with the pair
 // kernel, as fast as the bf16 weights; without the word loads and the decode
-// 203 us, so the MFMAs' rate on real data bounds it.
+// 203 us.  The MFMAs are busy 30 % of its cycles (T = 3001, Zipf), so they do not
+// bound it; real operands cost clock (zero ones: 271 -> 214 us back to back).
 template <int NBM>
 __device__ __forceinline__ void load_role_w4(const ExpertArgs &a, const UnitMap &map, int first, int stride, int nu,
                                              int lw, int lane, uint8_t *smem) {
