@@ -215,10 +215,11 @@ __device__ __forceinline__ void store_row(uint16_t *p, u32x4 v) { __builtin_nont
 // Those are lanes 0-3, 12-15, 20-23 and 24-27 of a 16-byte operand read (and the
 // other sixteen of 32), not consecutive ones: with (m >> 1) ^ (m >> 3 & 2), which
 // is conflict-free for consecutive lanes only, half of the LDS cycles were
-// conflicts (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE 0.50, now 0.02 in gate/up, 0.08
-// with the down epilogue, 0.30 with the W4 writes; times within 1 %: the LDS does
-// not bound these kernels).  The Gray code of m / 4 serves both groupings, in the operand reads
-// (consecutive rows, one chunk) and in the W4 loaders' writes (rows 8 q + 4 hb + i).
+// conflicts (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE 0.50).  The Gray code of m / 4
+// serves both groupings (consecutive rows, one chunk): 0.02 in gate/up, 0.08 with
+// the down epilogue; the W4 kernel, whose loaders write rows 8 q + 4 hb + i of one
+// chunk, keeps 0.30.  Times moved by less than 1 %: the LDS does not bound these
+// kernels.
 __device__ __forceinline__ int swz(int m) { return (((m >> 2) ^ (m >> 3)) & 3) << 1 | ((m >> 1) & 1); }
 // swz(8 j + lr) for lr < 8 is (lr >> 1) ^ swz8(j).
 __device__ __forceinline__ uint32_t swz8(int j) { return (uint32_t)(4 * ((j ^ (j >> 1)) & 1) | 2 * (j & 1)); }
